@@ -220,6 +220,7 @@ __global__ __launch_bounds__(256) void k_load_pos(const double* __restrict__ X, 
 }
 
 #include "od_kernels_pair.inc"
+#include "od_kernels_tile.inc"
 #include "od_kernels_step.inc"
 #include "od_kernels_trap.inc"
 #include "od_kernels_cell.inc"
@@ -277,6 +278,9 @@ struct od_ctx {
   double *sym_tp = nullptr, *sym_dg = nullptr, *rowD = nullptr, *sym_acc = nullptr;
   float* sym_sp = nullptr;
   std::vector<int> band_row, band_slot;
+  // wave tiles (k_pair_tile)
+  int tile = 0;
+  TilePlan tl;
   // cutoff mode: cell list; Gcut: flagged sources' share of the drift-state force;
   // sc_tp, sc_sp: partials of the symmetric cell kernel (FP32c)
   double* Gcut = nullptr;
@@ -405,7 +409,7 @@ static void free_ctx(od_ctx* c) {
                   c->slot_of, c->list_ion, c->err, c->rec, c->wg_tab, c->wg_base, c->sym_tp, c->sym_dg,
                   c->rowD, c->sym_sp, c->sym_acc, c->Gcut, c->scan_tsum, c->scan_toff, c->sc_tp, c->sc_sp, c->ckey[0], c->ckey[1], c->cval[0], c->cval[1], c->rs_hist,
                   c->rs_off, c->rs_total, c->cell_start, c->cell_chunks, c->item_off, c->items,
-                  c->n_items, c->spos};
+                  c->n_items, c->spos, c->tl.groups, c->tl.wg_group, c->tl.subs, c->tl.tp, c->tl.sp};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -421,6 +425,69 @@ static int dalloc(P** p, size_t bytes) {
   hipError_t e = hipMalloc((void**)p, bytes);
   if (e != hipSuccess) return set_err(OD_ERR_HIP, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   return OD_OK;
+}
+
+// (Re)builds the wave-tile plan *t; its old buffers are freed first.
+static int tile_build(TilePlan* t, const TileSims& sims, bool fp32) {
+  void* old[] = {t->groups, t->wg_group, t->subs, t->tp, t->sp};
+  for (void* q : old)
+    if (q) (void)hipFree(q);
+  *t = TilePlan();
+  tile_shape(sims, fp32, &t->mt, &t->nw);
+  const int gm = t->mt * t->nw;
+  const int64_t units = tile_units(sims, gm);
+  if (units > (1ll << 31) - 1) return set_err(OD_ERR_ARG, "wave tiles: too many units");
+  std::vector<TileGroup> groups;
+  std::vector<int4> subs;
+  int u = 0;
+  for (size_t m = 0; m < sims.count.size(); ++m) {
+    const int s0 = sims.first[m], s1 = s0 + sims.count[m], g0 = (int)groups.size();
+    for (int k = s0; k < s1; k += gm) {
+      groups.push_back({k, s1, u, (int)m});
+      u += s1 - k;
+    }
+    for (int k = s0; k < s1; ++k) subs.push_back(make_int4(k, g0 + (k - s0) / gm, g0, 0));
+  }
+  t->n_groups = (int)groups.size();
+  groups.push_back({0, 0, u, 0});
+  t->n_units = u;
+  t->n_sub = (int)subs.size();
+  t->per = std::max(1, (u + TILE_WGS - 1) / TILE_WGS);
+  t->n_wg = (u + t->per - 1) / t->per;
+  std::vector<int> wg(t->n_wg);
+  for (int b = 0, g = 0; b < t->n_wg; ++b) {
+    while (groups[g + 1].u0 <= b * t->per) ++g;
+    wg[b] = g;
+  }
+  const size_t segs = (size_t)t->n_wg + t->n_groups;
+  int rc = OD_OK;
+  if ((rc = dalloc(&t->groups, groups.size() * sizeof(TileGroup))) || (rc = dalloc(&t->wg_group, wg.size() * 4)) ||
+      (rc = dalloc(&t->subs, subs.size() * sizeof(int4))) || (rc = dalloc(&t->tp, segs * 192 * gm * 8)) ||
+      (rc = dalloc(&t->sp, (size_t)u * 192 * (fp32 ? 4 : 8))))
+    return rc;
+  HIPCHK(hipMemcpy(t->groups, groups.data(), groups.size() * sizeof(TileGroup), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(t->wg_group, wg.data(), wg.size() * 4, hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(t->subs, subs.data(), subs.size() * sizeof(int4), hipMemcpyHostToDevice));
+  return OD_OK;
+}
+
+// the tile kernel of plan t on pos (kernel coordinates)
+template <class T>
+static void launch_tile(const TilePlan& t, hipStream_t st, const DevParams* dP, const void* pos) {
+  using PV = typename Pos<T>::V;
+  void (*fn)(const DevParams*, const PV*, const TileGroup*, const int*, int, int, double*, T*);
+  if constexpr (std::is_same<T, float>::value)
+    fn = t.mt == 8 ? k_pair_tile<float, 8, 1, 4, 4> : k_pair_tile<float, 4, 1, 4, 4>;
+  else
+    fn = t.nw == 4 ? k_pair_tile<double, 4, 4, 1, 4> : k_pair_tile<double, 4, 1, 1, 4>;
+  hipLaunchKernelGGL(fn, dim3(t.n_wg), dim3(64 * t.nw), 0, st, dP, (const PV*)pos, (const TileGroup*)t.groups,
+                     (const int*)t.wg_group, t.n_units, t.per, t.tp, (T*)t.sp);
+}
+
+template <class T>
+static void launch_tile_reduce(const TilePlan& t, hipStream_t st, const DevParams* dP, int stride, double* F) {
+  hipLaunchKernelGGL(k_tile_reduce<T>, dim3(t.n_sub), dim3(256), 0, st, dP, (const TileGroup*)t.groups,
+                     (const int4*)t.subs, t.per, t.mt * t.nw, (const double*)t.tp, (const T*)t.sp, stride, F);
 }
 
 // launch geometry of the pair kernel
@@ -656,13 +723,49 @@ static int setup_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   return OD_OK;
 }
 
+// Whether a configuration without a schedule of its own runs the wave tiles:
+// FP64 whenever their partials fit; FP32 below TILE_FP32_SUBS sub-blocks of
+// 64 ions per simulation, above which the row groups of k_pair32_sym are
+// faster.  A configuration that fixes source chunks (j_split), blocks per
+// work-group, a variant or bands keeps the kernels those belong to.
+constexpr int TILE_FP32_SUBS = 4096;
+static bool tile_chosen(const od_config* cfg, const TileSims& sims) {
+  const bool fp32 = cfg->precision == OD_PREC_FP32C;
+  if (cfg->cutoff > 0.0 || cfg->pair_mode == OD_PAIR_ROWS || cfg->j_split > 0) return false;
+  if (!fp32) return tile_bytes(sims, false) <= TILE_MAX_BYTES;
+  if (cfg->pair_mode == OD_PAIR_SYM || cfg->sym_tile > 0 || cfg->sym_chunk > 0 || cfg->sym_band_mib > 0) return false;
+  const int most = *std::max_element(sims.count.begin(), sims.count.end());
+  return most < TILE_FP32_SUBS && tile_bytes(sims, true) <= TILE_MAX_BYTES;
+}
+
+static TileSims ctx_sims(const od_ctx* c) {
+  TileSims t;
+  t.first.push_back(0);
+  t.count.push_back((c->n + 63) / 64);
+  return t;
+}
+
+static int setup_k_pair32_sym(od_ctx* c, const od_config* cfg);
+
 static int setup_sym(od_ctx* c, const od_config* cfg) {
   c->sym = 0;
+  c->tile = 0;
+  const TileSims sims = ctx_sims(c);
+  if (tile_chosen(cfg, sims)) {
+    CHKRET(tile_build(&c->tl, sims, c->prec == OD_PREC_FP32C));
+    c->tile = 1;
+    return OD_OK;
+  }
+  return setup_k_pair32_sym(c, cfg);
+}
+
+// the schedule of k_pair32_sym, where the configuration runs it
+static int setup_k_pair32_sym(od_ctx* c, const od_config* cfg) {
   if (c->prec != OD_PREC_FP32C || cfg->pair_mode == OD_PAIR_ROWS || cfg->cutoff > 0.0) return OD_OK;
   const int T = c->n_pad / SYM_TB;
   const bool forced = cfg->pair_mode == OD_PAIR_SYM;
-  // automatic choice: symmetric from 2^15 ions (measured on MI355X, one step:
-  // 2^15 0.47 ms symmetric vs 0.62 ms rows, 2^14 0.30 vs 0.22 ms)
+  // without wave tiles: symmetric from 2^15 ions (measured on MI355X, one
+  // step: 2^15 0.47 ms symmetric vs 0.62 ms rows, 2^14 0.30 vs 0.22 ms)
   if (T < 2 || (!forced && c->n_pad < (1 << 15))) return OD_OK;
   const std::vector<int> be(T, T);
   int ch = sym_default_chunk(be, cfg->sym_chunk);
@@ -683,7 +786,8 @@ static int setup_sym(od_ctx* c, const od_config* cfg) {
     }
   }
   if ((rc = sym_build(c, be, ch, c->band_cap, sym_variants[var].rows)) ||
-      (rc = dalloc(&c->sym_dg, (size_t)3 * c->n_pad * 8)) || (rc = dalloc(&c->sym_acc, (size_t)3 * c->n_pad * 8)))
+      (!c->sym_dg && (rc = dalloc(&c->sym_dg, (size_t)3 * c->n_pad * 8))) ||
+      (!c->sym_acc && (rc = dalloc(&c->sym_acc, (size_t)3 * c->n_pad * 8))))
     return rc;
   c->sym_var = var;
   c->sym = 1;
@@ -802,6 +906,19 @@ static void mark(od_ctx* c, int stage) {
 static int launch_pair(od_ctx* c, const void* pi, const void* pj, double* F, bool timed) {
   const double L = 1.4426950408889634;
   const double C = c->cfg.kqq / (c->cfg.r_D_e * c->cfg.r_D_e);
+  if (c->tile && pi == pj) {
+    if (timed) HIPCHK(hipEventRecord(c->ev0, c->stream));
+    if (c->prec == OD_PREC_FP32C)
+      launch_tile<float>(c->tl, c->stream, c->dP, pj);
+    else
+      launch_tile<double>(c->tl, c->stream, c->dP, pj);
+    if (timed) HIPCHK(hipEventRecord(c->ev1, c->stream));
+    if (c->prec == OD_PREC_FP32C)
+      launch_tile_reduce<float>(c->tl, c->stream, c->dP, c->n_pad, F);
+    else
+      launch_tile_reduce<double>(c->tl, c->stream, c->dP, c->n_pad, F);
+    return OD_OK;
+  }
   if (c->sym && pi == pj) {
     const float a = (float)(c->cfg.r_0 / c->cfg.r_D_e * L), linv = (float)(1.0 / L);
     if (timed) HIPCHK(hipEventRecord(c->ev0, c->stream));
@@ -1378,7 +1495,7 @@ extern "C" int od_sym_choice(od_ctx* c, int32_t* sym_chunk, int32_t* sym_tile, i
 extern "C" int od_pair_info(od_ctx* c, int32_t* mode, int64_t* pairs_per_launch) {
   if (!c) return set_err(OD_ERR_ARG, "null context");
   const int64_t n = c->n;
-  if (mode) *mode = c->cut ? OD_PAIR_CELL : (c->sym ? OD_PAIR_SYM : OD_PAIR_ROWS);
+  if (mode) *mode = c->cut ? OD_PAIR_CELL : (c->sym || c->tile ? OD_PAIR_SYM : OD_PAIR_ROWS);
   if (c->cut) {
     if (pairs_per_launch) *pairs_per_launch = -1;  // data dependent: od_cutoff_pair_count
     return OD_OK;
@@ -1550,12 +1667,26 @@ extern "C" const char* od_build_info(void) { return "opendust_amd engine, gfx950
 // and can be fixed through od_config.sym_chunk and od_config.sym_tile.
 static const int kTuneChunks[] = {1, 2, 4, 8, 16, 32};
 
+// HIP-event time of `reps` evaluations on the context's stream
+template <class C, class F>
+static int time_evaluations(C* c, int reps, F&& evaluate, double* ms) {
+  HIPCHK(hipEventRecord(c->ev0, c->stream));
+  for (int r = 0; r < reps; ++r) evaluate();
+  HIPCHK(hipEventRecord(c->ev1, c->stream));
+  HIPCHK(hipEventSynchronize(c->ev1));
+  HIPCHK(hipGetLastError());
+  float t = 0.f;
+  HIPCHK(hipEventElapsedTime(&t, c->ev0, c->ev1));
+  *ms = t;
+  return OD_OK;
+}
+
 // band_cap: the band size schedules are built with (batches: unlimited, one
 // band).  Candidates whose partials exceed skip_cap in all (48 GB) are
 // skipped, which keeps tuning short; larger schedules keep their default.
 template <class C, class F>
 static int tune_sym(C* c, const std::vector<int>& be, int reps, F&& evaluate, int* chosen_ch, int* chosen_var,
-                    double band_cap, double skip_cap) {
+                    double band_cap, double skip_cap, double* best_of = nullptr) {
   double best_ms = 1e300;
   int best_ch = c->sym_ch, best_var = c->sym_var;
   struct Cand {
@@ -1578,14 +1709,9 @@ static int tune_sym(C* c, const std::vector<int>& be, int reps, F&& evaluate, in
     if (c->sym_ch != ch || c->sym_R != R) CHKRET(sym_build(c, be, ch, band_cap, R));
     c->sym_var = var;
     evaluate();  // warm-up
-    HIPCHK(hipEventRecord(c->ev0, c->stream));
-    for (int r = 0; r < reps; ++r) evaluate();
-    HIPCHK(hipEventRecord(c->ev1, c->stream));
-    HIPCHK(hipEventSynchronize(c->ev1));
-    HIPCHK(hipGetLastError());
-    float ms = 0.f;
-    HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-    cands.push_back({(double)ms, sym_bytes(be, ch, R), ch, var});
+    double ms = 0.0;
+    CHKRET(time_evaluations(c, reps, evaluate, &ms));
+    cands.push_back({ms, sym_bytes(be, ch, R), ch, var});
     if (ms < best_ms) {
       best_ms = ms;
       best_ch = ch;
@@ -1619,6 +1745,7 @@ static int tune_sym(C* c, const std::vector<int>& be, int reps, F&& evaluate, in
   c->sym_var = best_var;
   *chosen_ch = best_ch;
   *chosen_var = best_var;
+  if (best_of) *best_of = best_ms;
   return OD_OK;
 }
 
@@ -1681,15 +1808,32 @@ extern "C" int od_tune(od_ctx* c, int32_t reps, int32_t* sym_chunk, int32_t* sym
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
   }
-  if (c->sym) {
+  // wave tiles in FP32: k_pair32_sym (from 2^15 ions) replaces them only if
+  // its best schedule is faster
+  const bool tiles = c->tile && c->prec == OD_PREC_FP32C && c->n_pad >= (1 << 15);
+  if (c->sym || tiles) {
     if (!c->have_ions) return set_err(OD_ERR_STATE, "od_tune needs the ions (call od_set_ions first)");
     HIPCHK(hipSetDevice(c->dev));
     double* Fs = nullptr;
     CHKRET(dalloc(&Fs, (size_t)3 * c->n_pad * 8));
+    auto evaluate = [&]() { launch_pair(c, c->pj, c->pj, Fs, false); };
+    int rc = OD_OK;
+    double tile_ms = 1e300, sym_ms = 1e300;
+    if (tiles) {
+      evaluate();  // warm-up
+      rc = time_evaluations(c, reps, evaluate, &tile_ms);
+      c->tile = 0;
+      if (rc == OD_OK) rc = setup_k_pair32_sym(c, &c->cfg);
+    }
     const std::vector<int> be(c->n_blocks, c->n_blocks);
-    const int rc = tune_sym(c, be, reps, [&]() { launch_pair(c, c->pj, c->pj, Fs, false); }, &chosen, &var,
-                            c->band_cap, SYM_BAND_BYTES);
+    if (rc == OD_OK) rc = tune_sym(c, be, reps, evaluate, &chosen, &var, c->band_cap, SYM_BAND_BYTES, &sym_ms);
     (void)hipFree(Fs);
+    if (tiles && (rc != OD_OK || tile_ms <= sym_ms)) {
+      c->tile = 1;
+      c->sym = 0;
+      chosen = 0;
+      var = -1;
+    }
     if (rc != OD_OK) return rc;
     // the ion-ion force of the current positions, with the chosen schedule
     CHKRET(load_positions(c, c->X, c->pi, c->pj));
@@ -1711,6 +1855,11 @@ extern "C" int od_batch_tune(od_batch* b, int32_t reps, int32_t* sym_chunk, int3
     if (b->stale)
       hipLaunchKernelGGL(k_batch_load_pos<float>, dim3(b->nb), dim3(256), 0, b->stream, b->dP, b->blk_sim, b->X,
                          (float4*)b->pi, (float4*)b->pj);
+    if (b->tile) {
+      // the schedules tuned here are k_pair32_sym's: it replaces the wave tiles
+      if (b->blk_end_host.empty()) CHKRET(batch_setup_sym(b));
+      b->tile = 0;
+    }
     double* Fs = nullptr;
     CHKRET(dalloc(&Fs, (size_t)3 * b->n_tot * 8));
     const int rc = tune_sym(b, b->blk_end_host, reps, [&]() { batch_pair<float>(b, false, Fs); }, &chosen, &var,

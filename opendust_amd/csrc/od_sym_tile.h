@@ -287,16 +287,16 @@ __device__ __forceinline__ float wave_ror1(float v) {
 // cell kernel with 2 target sub-blocks ran slower with it, 52.2 -> 57.0 ms
 // at 2^22, and does without.
 // ls: this lane's entry ls + lane + 64.  (bx, by, bz): added to.
-template <int MT, int CUT, bool PF = false>
+template <int MT, int CUT, bool PF = false, int UN = 16>
 __device__ __forceinline__ void sym_tile_lds(SymT<MT>& T, const float4* ls, float& bx, float& by, float& bz,
                                              const SymLaw& L) {
   const float eps = vgpr(EPS32);
   // PF: the read after the last step, ls[-64], is the lane's own entry
   // ls[lane] (in bounds, unused)
   float4 qn = ls[0];
-  for (int s0 = 0; s0 < 64; s0 += 16) {
+  for (int s0 = 0; s0 < 64; s0 += UN) {
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
+    for (int s = 0; s < UN; ++s) {
       float4 q;
       if constexpr (PF) {
         q = qn;

@@ -1,0 +1,151 @@
+"""The wave-tile all-pairs kernel (even split of 64-ion tiles) and the FP64
+pair law's own elementary functions."""
+
+import contextlib
+import io
+
+import numpy as np
+import pytest
+
+from conftest import say
+
+pytestmark = pytest.mark.gpu
+
+
+def _setup(N, precision, np_seed=5):
+    from opendust_amd import workloads
+
+    with contextlib.redirect_stdout(io.StringIO()):
+        od = workloads.single_dust(N=N, n=3, precision=precision, seed=3)
+        return workloads.prepare(od, alpha=workloads.synthetic_alpha(od), np_seed=np_seed, precision=precision)
+
+
+def _forces(cfg, x, mode):
+    from opendust_amd import engine
+
+    cfg = engine.Config.from_buffer_copy(cfg)
+    cfg.pair_mode = mode
+    e = engine.Engine(cfg)
+    f = e.pair_forces(x)
+    info = e.pair_info()
+    e.close()
+    return f, info
+
+
+# edges of a 64-ion sub-block, of a target group (4 and 8 sub-blocks, 16 with
+# 4 waves), the changes of shape at 2^15 (FP32) and 2^17 (FP64) ions, several
+# work-groups per group and several groups per work-group
+@pytest.mark.parametrize("precision,N", [(p, n) for p in ("fp64", "fp32c") for n in (
+    1, 2, 63, 64, 65, 255, 256, 257, 513, 4095, 5000)] + [
+    ("fp32c", 32704), ("fp32c", 32705), ("fp32c", 70001), ("fp32c", 262080), ("fp64", 40001), ("fp64", 131009)])
+def test_wave_tiles_vs_oracle_or_rows(oracle_lib, precision, N):
+    """Small sizes against the oracle (the bounds of the other pair kernels);
+    larger ones against the row kernel in the same precision, with twice the
+    arithmetic bound, since both sides carry it."""
+    from opendust_amd import engine
+
+    cfg, x0, _ = _setup(N, precision)
+    say("wave tiles", precision, "N", N)
+    f, info = _forces(cfg, x0, engine.PAIR_AUTO)
+    assert info == (engine.PAIR_SYM, N * (N - 1))
+    if N <= 5000:
+        ref = oracle_lib.pair_forces(cfg, x0)
+        rel_i, rel_rms, rel = (1e-11, 1e-13, 1e-11) if precision == "fp64" else (1e-4, 1e-5, 1e-5)
+    else:
+        ref, info = _forces(cfg, x0, engine.PAIR_ROWS)
+        assert info[0] == engine.PAIR_ROWS
+        rel_i, rel_rms, rel = (1e-11, 1e-13, 1e-11) if precision == "fp64" else (2e-5, 2e-6, 4e-6)
+    fn = np.linalg.norm(ref, axis=1)
+    rms = np.sqrt(np.mean(fn ** 2))
+    err = np.linalg.norm(f - ref, axis=1)
+    say("  norm-wise", np.linalg.norm(f - ref) / max(np.linalg.norm(ref), 1e-300))
+    assert np.all(err <= rel_i * fn + rel_rms * rms)
+    assert np.linalg.norm(f - ref) <= rel * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+def test_wave_tiles_batch_equals_single(precision):
+    """Simulations of a batch whose sizes end inside a sub-block and a group:
+    the same forces as each alone (same groups, so the same sums up to where
+    work-groups split them), seen through one step's velocities."""
+    from opendust_amd import engine
+
+    sizes = [1, 64, 700, 2049, 5000]
+    setups = [_setup(n, precision, np_seed=20 + i) for i, n in enumerate(sizes)]
+    for s, (cfg, _, _) in enumerate(setups):
+        cfg.sim_id = s
+    say("wave tiles, batch", precision, sizes)
+    b = engine.Batch([c for c, _, _ in setups])
+    for s, (_, x, v) in enumerate(setups):
+        b.set_ions(s, x, v)
+    b.run(2)
+    for s, (cfg, x, v) in enumerate(setups):
+        e = engine.Engine(cfg)
+        e.set_ions(x, v)
+        e.run(2)
+        xs, vs = e.get_ions()
+        e.close()
+        xb, vb = b.get_ions(s)
+        tol = 1e-12 if precision == "fp64" else 1e-6
+        assert np.max(np.abs(xb - xs)) <= tol * cfg.R
+        assert np.max(np.abs(vb - vs)) <= tol * np.max(np.abs(vs))
+    b.close()
+
+
+def test_tune_keeps_or_replaces_wave_tiles():
+    """od_tune on a context that runs wave tiles: (0, 0) and the same forces
+    when they stay, else a k_pair32_sym schedule within the FP32c bound."""
+    from opendust_amd import engine
+
+    cfg, x0, v0 = _setup(32768, "fp32c")
+    e = engine.Engine(cfg)
+    e.set_ions(x0, v0)
+    f0 = e.pair_forces(x0)
+    say("tune over wave tiles")
+    chosen = e.tune(2)
+    f1 = e.pair_forces(x0)
+    assert e.sym_choice() == chosen
+    if chosen == (0, 0):
+        assert np.array_equal(f0, f1)
+    else:
+        assert np.linalg.norm(f1 - f0) <= 4e-6 * np.linalg.norm(f0)
+    e.run(4, engine.RUN_GRAPH)
+    e.close()
+
+
+def test_fp64_pair_law_over_its_range():
+    """Two ions from 1e-6 to 600 r_D_e apart, FP64 (rsqrt, exp and 1/x of the
+    kernels' own), against numpy: about 10 roundings, and the rounding of the
+    distance r enters exp(-r) as r times its relative error."""
+    from opendust_amd import engine
+
+    cfg, _, _ = _setup(64, "fp64")
+    cfg = engine.Config.from_buffer_copy(cfg)
+    cfg.n_ions = 2
+    cfg.n_dust = 0
+    lam, a = cfg.r_D_e, cfg.r_0 / cfg.r_D_e
+    say("FP64 pair law")
+    for mode in (engine.PAIR_AUTO, engine.PAIR_ROWS):
+        cfg.pair_mode = mode
+        e = engine.Engine(cfg)
+        for d in np.geomspace(1e-6, 600.0, 60):
+            x = np.array([[0.0, 0.0, 0.0], [0.6 * d * lam, -0.64 * d * lam, 0.48 * d * lam]])
+            r = np.linalg.norm(x[1] / lam)
+            want = cfg.kqq / lam ** 2 * np.exp(-r) / (r + a) * (1 + 1 / (r + a)) * (-x[1] / lam / r)
+            f = e.pair_forces(x)
+            tol = 4e-15 + 1e-15 * r
+            assert np.linalg.norm(f[0] - want) <= tol * np.linalg.norm(want), d
+            assert np.linalg.norm(f[1] + want) <= tol * np.linalg.norm(want), d
+        e.close()
+
+
+@pytest.mark.parametrize("n_r,n_h,n_mc", [(1, 1, 1), (2, 4, 255), (3, 5, 257), (2, 6, 65536), (1, 11, 65537)])
+def test_trap_grid_edges_vs_oracle(oracle_lib, n_r, n_h, n_mc):
+    """Heights around the tile of five, samples around a block and a chunk."""
+    from opendust_amd import engine
+
+    rho, h = np.linspace(0, 3.0, n_r), np.linspace(0, 2.5, n_h)
+    say("trap grid", n_r, n_h, n_mc)
+    g = engine.trap_potential_grid(3.0, 5.0, rho, h, n_mc, 17)
+    o = oracle_lib.trap_grid(3.0, 5.0, rho, h, n_mc, 17)
+    assert g.shape == (n_r, n_h) and np.max(np.abs(g - o) / np.abs(o)) <= 1e-12
