@@ -1625,8 +1625,9 @@ extern "C" int od_trap_potential_grid(int32_t device, double R, double H, int32_
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_trap_samples, dim3((unsigned)((n_mc + 255) / 256)), dim3(256), 0, 0, R, H, seed, n_mc, xs,
                        ys, zs);
-    hipLaunchKernelGGL(k_trap_grid, dim3(n_gp * n_chunks), dim3(256), 0, 0, drho, dh, n_h, xs, ys, zs, n_mc, chunk,
-                       n_chunks, part);
+    const int n_tiles = n_r * ((n_h + TRAP_H - 1) / TRAP_H);
+    hipLaunchKernelGGL(k_trap_grid, dim3(n_tiles * n_chunks), dim3(256), 0, 0, drho, dh, n_h, n_tiles, xs, ys, zs,
+                       n_mc, chunk, n_chunks, part);
     hipLaunchKernelGGL(k_trap_finish, dim3((n_gp + 255) / 256), dim3(256), 0, 0, part, n_gp, n_chunks, (double)n_mc,
                        dout);
     e = hipGetLastError();
