@@ -226,6 +226,24 @@ __device__ __forceinline__ void pair32_cut(float xi, float yi, float zi, float x
   az = __builtin_fmaf(h, dz, az);
 }
 
+// the truncated FP64 law's h, by selection (no branch)
+template <bool SW>
+__device__ __forceinline__ double pair64_cut_h(double r2, double rho0, double rc, double rs, double invw) {
+  const double y = rsqrt64(r2);
+  const double r = r2 * y;
+  const double e = exp_neg64(r);
+  const double z = recip64(r + rho0);
+  const double yz = y * z;
+  double h = e * fma(yz, z, yz);
+  if constexpr (SW) {
+    const double x = fmin(fmax((r - rs) * invw, 0.0), 1.0);
+    const double x2 = x * x, omx = 1.0 - x;
+    const double S = fma(x2 * x, fma(x, fma(x, -6.0, 15.0), -10.0), 1.0);
+    h = fma(h, S, e * yz * (30.0 * x2 * omx * omx * invw));
+  }
+  return (r < rc) ? h : 0.0;
+}
+
 __device__ __forceinline__ void pair64_cut(double xi, double yi, double zi, double xj, double yj, double zj,
                                            double rho0, bool sw, double rc, double rs, double invw, double& ax,
                                            double& ay, double& az) {

@@ -296,6 +296,12 @@ struct od_ctx {
       *cell_chunks = nullptr, *item_off = nullptr, *n_items = nullptr;
   int2* items = nullptr;
   void* spos = nullptr;
+  // even split of the cell list (k_cell_list): entries, first units, partials
+  int list = 0, cl_cap = 0, n_entries = 0, item_len = 64;
+  int2* cl_rng = nullptr;
+  int *cl_cnt = nullptr, *cl_u0 = nullptr, *cl_total = nullptr;
+  double* cl_tp = nullptr;
+  void* cl_sp = nullptr;
 };
 
 static int fill_params(const od_config* c, int n_pad, DevParams* P) {
@@ -409,7 +415,8 @@ static void free_ctx(od_ctx* c) {
                   c->slot_of, c->list_ion, c->err, c->rec, c->wg_tab, c->wg_base, c->sym_tp, c->sym_dg,
                   c->rowD, c->sym_sp, c->sym_acc, c->Gcut, c->scan_tsum, c->scan_toff, c->sc_tp, c->sc_sp, c->ckey[0], c->ckey[1], c->cval[0], c->cval[1], c->rs_hist,
                   c->rs_off, c->rs_total, c->cell_start, c->cell_chunks, c->item_off, c->items,
-                  c->n_items, c->spos, c->tl.groups, c->tl.wg_group, c->tl.subs, c->tl.tp, c->tl.sp};
+                  c->n_items, c->spos, c->tl.groups, c->tl.wg_group, c->tl.subs, c->tl.tp, c->tl.sp, c->cl_rng, c->cl_cnt,
+                  c->cl_u0, c->cl_total, c->cl_tp, c->cl_sp};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -681,6 +688,40 @@ static int sym_default_chunk(const std::vector<int>& be, int configured) {
   return ch;
 }
 
+// Units of k_cell_list for ions spread evenly over the cylinder: per group and
+// set the column's ions in the slab reach and the group's own length, in
+// 64-ion chunks, one more for the remainder.
+static double cell_list_units(const od_ctx* c, const od_config* cfg) {
+  const double pi = 3.141592653589793;
+  const double w = cfg->cutoff / 4.0, h = cfg->cutoff / 16.0;
+  const double line = c->n / (pi * cfg->R * cfg->R * cfg->H) * w * w;  // ions per length of a column
+  const double len = std::min(cfg->H, CL_G / line);
+  double per_group = 0.0;
+  for (int k = 0; k < CC_NSET; ++k) {
+    int dx = 0, dy = 0;
+    if (k < CC_NFWD) cc_fwd(k, dx, dy);
+    per_group += std::min(cfg->H, (2 * cc_nbz(dx, dy) + 1) * h + len) * line / 64.0 + 1.0;
+  }
+  return ((double)c->n / CL_G + c->n_cols) * per_group;
+}
+
+// Whether the context runs k_cell_list: where its partials, at twice the even
+// spread's units, fit CELL_LIST_MAX_BYTES; in FP32c only where the column
+// kernel's waves (one per column and set, at most) are too few to fill the
+// chip, and not if the configuration fixes a variant of that kernel.  Force
+// evaluation, column kernel -> list: 131072 ions in 64 columns 5.37 -> 1.81
+// ms, 16384 0.38 -> 0.23; with 1600 columns 32768 ions 0.21 -> 0.24, 2^20 5.51
+// -> 5.61, 2^22 53.2 -> 52.6.
+constexpr double CELL_LIST_MAX_BYTES = 24e9;
+constexpr int CELL_COLUMN_WAVES = 16384;
+static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, int* cap) {
+  const double units = 2.0 * cell_list_units(c, cfg) + 4096.0;
+  const bool fp32 = c->prec == OD_PREC_FP32C;
+  *cap = (int)std::min(units, 1e9);
+  if (fp32 && (cfg->sym_tile > 0 || c->n_cols * CC_NSET >= CELL_COLUMN_WAVES)) return false;
+  return units * 192.0 * (fp32 ? 4.0 : 8.0) <= CELL_LIST_MAX_BYTES;
+}
+
 static int setup_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   c->cut = 0;
   if (!(cfg->cutoff > 0.0)) return OD_OK;
@@ -697,7 +738,10 @@ static int setup_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   c->rs_passes = 1;
   while (c->rs_passes < 4 && ((uint64_t)c->n_cells >> (8 * c->rs_passes)) != 0) ++c->rs_passes;
   c->rs_nblk = (c->n_pad + RS_ITEMS - 1) / RS_ITEMS;
-  c->max_items = c->n_pad / 64 + c->n_cols + 1;
+  c->list = cell_list_chosen(c, cfg, &c->cl_cap) ? 1 : 0;
+  c->item_len = c->list ? CL_G : 64;
+  c->max_items = c->n_pad / c->item_len + c->n_cols + 1;
+  c->n_entries = c->list ? c->max_items * CC_NSET : 0;
   const size_t np = c->n_pad;
   int rc = OD_OK;
   if ((rc = dalloc(&c->ckey[0], np * 4)) || (rc = dalloc(&c->ckey[1], np * 4)) || (rc = dalloc(&c->cval[0], np * 4)) ||
@@ -711,8 +755,18 @@ static int setup_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
     return rc;
   c->skey = c->ckey[c->rs_passes & 1];
   c->sval = c->cval[c->rs_passes & 1];
-  const size_t n_tiles = (std::max<size_t>((size_t)256 * c->rs_nblk, (size_t)c->n_cols + 1) + 1023) / 1024;
+  const size_t n_scan = std::max({(size_t)256 * c->rs_nblk, (size_t)c->n_cols + 1, (size_t)c->n_entries + 1});
+  const size_t n_tiles = (n_scan + 1023) / 1024;
   if ((rc = dalloc(&c->scan_tsum, n_tiles * 4)) || (rc = dalloc(&c->scan_toff, n_tiles * 4))) return rc;
+  c->sc_var = CC_DEFAULT;
+  if (c->list) {
+    const size_t ne = (size_t)c->n_entries + 1;
+    if ((rc = dalloc(&c->cl_rng, ne * sizeof(int2))) || (rc = dalloc(&c->cl_cnt, ne * 4)) ||
+        (rc = dalloc(&c->cl_u0, ne * 4)) || (rc = dalloc(&c->cl_total, 4)) ||
+        (rc = dalloc(&c->cl_tp, ((size_t)CL_WAVES + c->max_items) * 3 * CL_G * 8)) ||
+        (rc = dalloc(&c->cl_sp, (size_t)c->cl_cap * 192 * (c->prec == OD_PREC_FP32C ? 4 : 8))))
+      return rc;
+  }
   if (c->prec == OD_PREC_FP32C) {
     if ((rc = dalloc(&c->sc_tp, (size_t)CC_NSET * 3 * np * 8)) ||
         (rc = dalloc(&c->sc_sp, (size_t)CC_NSET * 3 * np * 4)))
@@ -1004,12 +1058,17 @@ static int build_cells_t(od_ctx* c, const double* X, const uint32_t* flags, cons
   hipLaunchKernelGGL(k_cell_starts, dim3(nc / 256 + 1), dim3(256), 0, c->stream, c->skey, np, nc, c->cell_start);
   const int gc = (c->n_cols + 255) / 256;
   hipLaunchKernelGGL(k_cell_chunks, dim3(gc), dim3(256), 0, c->stream, c->cell_start, c->n_cols, c->nz,
-                     c->cell_chunks);
+                     c->item_len, c->cell_chunks);
   launch_scan(c, c->cell_chunks, c->n_cols, c->item_off, c->n_items);
   hipLaunchKernelGGL(k_cell_items, dim3(gc), dim3(256), 0, c->stream, c->cell_chunks, c->item_off, c->n_cols,
                      c->items);
   hipLaunchKernelGGL(k_cell_gather<T>, dim3(nb), dim3(256), 0, c->stream, c->skey, c->sval, np, nc,
                      (const PV*)pos, (PV*)c->spos);
+  if (c->list) {
+    hipLaunchKernelGGL(k_cell_ranges, dim3(c->n_entries / 256 + 1), dim3(256), 0, c->stream, c->dP, c->skey,
+                       c->cell_start, c->items, c->n_items, c->n_entries, c->cl_rng, c->cl_cnt);
+    launch_scan(c, c->cl_cnt, c->n_entries + 1, c->cl_u0, c->cl_total);
+  }
   return OD_OK;
 }
 
@@ -1030,21 +1089,30 @@ static int launch_forces_t(od_ctx* c, const double* X, const void* pos, const ui
   const int grid = std::max(1, std::min(4096, c->max_items / 4 + 1));
   const bool sw = c->cfg.switch_dist > 0.0 && c->cfg.switch_dist < c->cfg.cutoff;
   if (timed) HIPCHK(hipEventRecord(c->ev0, c->stream));
+  const int* n_units = c->list ? c->cl_total : nullptr;
+  if (c->list) {
+    // the kernels after these two return at once unless the units overflow
+    hipLaunchKernelGGL((sw ? k_cell_list<T, 2> : k_cell_list<T, 1>), dim3(CL_WAVES), dim3(64), 0, c->stream, c->dP,
+                       (const PV*)c->spos, c->skey, c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries,
+                       n_units, c->cl_cap, c->cl_tp, (T*)c->cl_sp);
+    hipLaunchKernelGGL(k_cell_list_reduce<T>, dim3(c->n_pad / 256), dim3(256), 0, c->stream, c->dP, c->skey, c->sval,
+                       c->cell_start, c->item_off, c->cl_rng, c->cl_u0, n_units, c->cl_cap, CL_WAVES,
+                       (const double*)c->cl_tp, (const T*)c->cl_sp, F);
+  }
   if constexpr (std::is_same<T, float>::value) {
     // symmetric: forward neighbour columns and the own column, per-ion reduction
     const float4* sp4 = (const float4*)c->spos;
     const dim3 g(c->n_cols * CC_NSET);
     const int ki = c->sc_var * 2 + (sw ? 1 : 0);
-    hipLaunchKernelGGL(cell_sym_kernels[ki], g, dim3(64), 0, c->stream, c->dP, sp4, c->skey, c->cell_start, c->sc_tp,
-                       c->sc_sp);
+    hipLaunchKernelGGL(cell_sym_kernels[ki], g, dim3(64), 0, c->stream, c->dP, sp4, c->skey, c->cell_start, n_units,
+                       c->cl_cap, c->sc_tp, c->sc_sp);
     hipLaunchKernelGGL(k_symcol_reduce, dim3(c->n_pad / 256), dim3(256), 0, c->stream, c->dP, c->skey, c->sval,
-                       c->cell_start, 64 * cell_variant_mt[c->sc_var], (const double*)c->sc_tp, (const float*)c->sc_sp, F);
-  } else if (sw) {
-    hipLaunchKernelGGL((k_pair_cell<T, 1>), dim3(grid), dim3(256), 0, c->stream, c->dP, (const PV*)c->spos,
-                       c->skey, c->sval, c->cell_start, c->items, c->n_items, F);
+                       c->cell_start, 64 * cell_variant_mt[c->sc_var], n_units, c->cl_cap, (const double*)c->sc_tp,
+                       (const float*)c->sc_sp, F);
   } else {
-    hipLaunchKernelGGL((k_pair_cell<T, 0>), dim3(grid), dim3(256), 0, c->stream, c->dP, (const PV*)c->spos,
-                       c->skey, c->sval, c->cell_start, c->items, c->n_items, F);
+    hipLaunchKernelGGL((sw ? k_pair_cell<T, 1> : k_pair_cell<T, 0>), dim3(grid), dim3(256), 0, c->stream, c->dP,
+                       (const PV*)c->spos, c->skey, c->sval, c->cell_start, c->items, c->n_items, c->item_len / 64,
+                       n_units, c->cl_cap, F);
   }
   if (timed) HIPCHK(hipEventRecord(c->ev1, c->stream));
   return OD_OK;
@@ -1387,7 +1455,8 @@ static int64_t cell_candidates(const od_ctx* c, const std::vector<int>& cs, cons
     const int cA = A * nz, a0 = cs[cA], a1 = cs[cA + nz];
     if (a0 == a1) continue;
     const int ax = A % nx, ay = A / nx;
-    if (c->prec == OD_PREC_FP32C) {
+    if (c->prec == OD_PREC_FP32C || c->list) {
+      // k_cell_list's units cover what variant 5 of the column kernel does
       const int MTv = cell_variant_mt[c->sc_var];
       const bool split = cell_variant_split[c->sc_var];
       const int G = 64 * MTv;
@@ -1458,10 +1527,10 @@ extern "C" int od_cutoff_pair_count(od_ctx* c, int64_t* in_range, int64_t* candi
   if (e == hipSuccess) {
     if (c->prec == OD_PREC_FP32C)
       hipLaunchKernelGGL(k_cell_pair_count<float>, dim3(grid), dim3(256), 0, c->stream, c->dP,
-                         (const float4*)c->spos, c->skey, c->cell_start, c->items, c->n_items, d);
+                         (const float4*)c->spos, c->skey, c->cell_start, c->items, c->n_items, c->item_len / 64, d);
     else
       hipLaunchKernelGGL(k_cell_pair_count<double>, dim3(grid), dim3(256), 0, c->stream, c->dP,
-                         (const double4*)c->spos, c->skey, c->cell_start, c->items, c->n_items, d);
+                         (const double4*)c->spos, c->skey, c->cell_start, c->items, c->n_items, c->item_len / 64, d);
     e = hipGetLastError();
   }
   std::vector<int> cs(c->n_cells + 1);
@@ -1482,7 +1551,7 @@ extern "C" int od_sym_choice(od_ctx* c, int32_t* sym_chunk, int32_t* sym_tile, i
   if (c->cut && c->prec == OD_PREC_FP32C) {
     // symmetric cell kernel: no source blocks, the variant 1 .. CC_N_VARIANTS
     if (sym_chunk) *sym_chunk = 0;
-    if (sym_tile) *sym_tile = c->sc_var + 1;
+    if (sym_tile) *sym_tile = c->list ? 0 : c->sc_var + 1;
     if (bands) *bands = 0;
     return OD_OK;
   }
@@ -1775,9 +1844,11 @@ static int tune_cells(od_ctx* c, int reps, int* chosen_var) {
   CHKRET(dalloc(&Fs, (size_t)3 * c->n_pad * 8));
   int rc = load_positions(c, c->X, c->pi, c->pj);
   double best_ms = 1e300;
-  int best = c->sc_var;
-  for (int v = 0; v < CC_N_VARIANTS && rc == OD_OK; ++v) {
-    c->sc_var = v;
+  const int had_list = c->list;
+  int best = had_list ? -1 : c->sc_var;
+  for (int v = had_list ? -1 : 0; v < CC_N_VARIANTS && rc == OD_OK; ++v) {
+    c->list = v < 0 ? 1 : 0;
+    c->sc_var = v < 0 ? CC_DEFAULT : v;
     rc = launch_forces(c, c->X, c->pj, nullptr, Fs, false);  // warm-up
     if (rc == OD_OK && hipEventRecord(c->ev0, c->stream) != hipSuccess) rc = set_err(OD_ERR_HIP, "hipEventRecord");
     for (int r = 0; r < reps && rc == OD_OK; ++r) rc = launch_forces(c, c->X, c->pj, nullptr, Fs, false);
@@ -1791,7 +1862,8 @@ static int tune_cells(od_ctx* c, int reps, int* chosen_var) {
     }
   }
   (void)hipFree(Fs);
-  c->sc_var = best;
+  c->list = best < 0 ? 1 : 0;
+  c->sc_var = best < 0 ? CC_DEFAULT : best;
   *chosen_var = best;
   return rc;
 }

@@ -1,0 +1,90 @@
+"""The even-split cell-list force (k_cell_list) where it can go wrong: few
+columns, groups and chunks that end inside a column, empty columns, clusters
+that overflow its buffer, and the grid it bins into."""
+
+import contextlib
+import io
+
+import numpy as np
+import pytest
+
+from conftest import say
+
+pytestmark = pytest.mark.gpu
+
+
+def _setup(N, precision, rc, rs, R=3.0, H=6.0, np_seed=2):
+    from opendust_amd import workloads
+
+    with contextlib.redirect_stdout(io.StringIO()):
+        od = workloads.single_dust(N=N, n=3, precision=precision, seed=4, R=R, H=H)
+        cfg, x0, v0 = workloads.prepare(od, alpha=workloads.synthetic_alpha(od), np_seed=np_seed, precision=precision)
+    cfg.cutoff = rc * cfg.r_D_e
+    cfg.switch_dist = 0.0 if rs is None else rs * cfg.r_D_e
+    return cfg, x0, v0
+
+
+def _check(oracle_lib, cfg, x0, precision):
+    """Forces, cells and order of one evaluation against the oracle: the bounds
+    of the other cutoff tests, FP32c on the rounded positions, a pair at the
+    rounding of a hard cutoff allowed on either side."""
+    from oracle.oracle import fp32c_rounded_positions
+
+    from opendust_amd import engine
+
+    e = engine.Engine(cfg)
+    f = e.pair_forces(x0)
+    cell, order, dims = e.cells()
+    f2 = e.pair_forces(x0)
+    e.close()
+    assert np.array_equal(f, f2)
+    if precision == "fp64":
+        ref, edge = oracle_lib.pair_forces(cfg, x0), np.zeros(len(x0))
+        rel_i, rel_rms = 1e-11, 1e-13
+    else:
+        xr = fp32c_rounded_positions(cfg, x0)
+        ref, edge = oracle_lib.pair_forces(cfg, xr), oracle_lib.cut_edge_count(cfg, xr, 1e-6)
+        rel_i, rel_rms = 1e-5, 1e-6
+    fn = np.linalg.norm(ref, axis=1)
+    rms = np.sqrt(np.mean(fn ** 2))
+    err = np.linalg.norm(f - ref, axis=1)
+    f_cut = oracle_lib.cut_force_at_cutoff(cfg) if cfg.switch_dist <= 0.0 else 0.0
+    bound = rel_i * fn + rel_rms * rms + edge * f_cut * 1.001
+    say("  worst per-ion error / bound", float(np.max(err / np.maximum(bound, 1e-300))))
+    assert np.all(err <= bound)
+    want = np.array([oracle_lib.cell_of(cfg, xi)[0] for xi in x0])
+    assert dims == oracle_lib.cell_of(cfg, x0[0])[1]
+    assert np.array_equal(cell, want)
+    assert np.array_equal(order, np.lexsort((np.arange(len(want)), want)))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+@pytest.mark.parametrize("N,rc,rs", [(1, 2.0, None), (64, 2.0, None), (129, 3.2, 3.0), (2500, 1.0, None),
+                                     (2500, 3.2, 3.0), (6001, 2.0, 1.5), (6001, 9.0, None)])
+def test_cell_list_sizes_vs_oracle(oracle_lib, precision, N, rc, rs):
+    cfg, x0, _ = _setup(N, precision, rc, rs)
+    say("cell list", precision, "N", N, "rc", rc, "rs", rs)
+    _check(oracle_lib, cfg, x0, precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+@pytest.mark.parametrize("shape", ["cluster", "two_slabs", "line"])
+def test_cell_list_uneven_ions_vs_oracle(oracle_lib, precision, shape):
+    """Ions far from evenly spread.  cluster: all in a ball of half the cutoff
+    (every pair interacts; the units exceed the buffer, so the fallback
+    kernels compute the force); two_slabs: the middle of every column empty,
+    so a group spans the gap; line: one column holds everything."""
+    cfg, x0, _ = _setup(4000, precision, 1.0, None, R=3.0, H=30.0)
+    rng = np.random.RandomState(5)
+    lam = cfg.r_D_e
+    if shape == "cluster":
+        d = rng.normal(size=x0.shape)
+        x0 = d / np.linalg.norm(d, axis=1)[:, None] * (0.5 * lam * rng.uniform(size=len(x0)) ** (1 / 3))[:, None]
+    elif shape == "two_slabs":
+        x0[:, 2] = np.where(np.arange(len(x0)) % 2, 14.0, -14.0) * lam + rng.uniform(-0.4, 0.4, len(x0)) * lam
+        x0[:50, 2] = rng.uniform(-14.0, 14.0, 50) * lam
+    else:
+        x0[:, 0] = 0.05 * lam + 0.01 * lam * rng.uniform(size=len(x0))
+        x0[:, 1] = 0.05 * lam + 0.01 * lam * rng.uniform(size=len(x0))
+    say("cell list, uneven ions", shape, precision)
+    _check(oracle_lib, cfg, x0, precision)
