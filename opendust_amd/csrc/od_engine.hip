@@ -75,6 +75,8 @@ static int scratch_address(int dev, double** out);
 // ---------------------------------------------------------------------------
 // device parameters (one copy per context, read-only in kernels)
 // ---------------------------------------------------------------------------
+constexpr int CC_MAX_FWD = 63;  // forward column offsets of a cell grid, at most
+
 struct DevParams {
   ExtParams ext;
   int n, n_pad, n_dust, distribution, use_bottom;
@@ -98,6 +100,11 @@ struct DevParams {
   // cell grid (nm): columns of col_w in x and y, slabs of slab_h in z
   double col_w, slab_h;
   int nx, ny, nz, n_cells;
+  int n_fwd;             // forward column offsets
+  int off[CC_MAX_FWD + 1];  // dx | dy << 8 | slab reach << 16: the forward offsets, then the own column
+  // the grid od_get_cells reports (columns cutoff/4, slabs cutoff/16)
+  double rc4_w, rc4_h;
+  int rc4_nx, rc4_nz, rc4_cells;
   uint64_t thr_top, thr_side, thr_coll;
   int dust_method[OD_MAX_DUST];
   double si_k, si_e, si_q_s, si_lam, si_dt, si_kB, si_Te, si_Tn, si_E;
@@ -232,6 +239,12 @@ __global__ __launch_bounds__(256) void k_load_pos(const double* __restrict__ X, 
 // Batches run one band.
 constexpr double SYM_BAND_BYTES = 48e9;
 
+// Cell grid of the cutoff forces: columns 2 cutoff / p2 wide in x and y, slabs
+// cutoff / q high in z.
+struct CellGrid {
+  int p2 = 8, q = 16;
+};
+
 // ---------------------------------------------------------------------------
 // context
 // ---------------------------------------------------------------------------
@@ -298,13 +311,41 @@ struct od_ctx {
   void* spos = nullptr;
   // even split of the cell list (k_cell_list): entries, first units, partials
   int list = 0, cl_cap = 0, n_entries = 0, item_len = 64;
+  CellGrid grid;
+  int n_set = 0;                  // forward column offsets + 1
+  uint32_t* rc4_cell = nullptr;   // od_get_cells' cells, where the grid is another
   int2* cl_rng = nullptr;
   int *cl_cnt = nullptr, *cl_u0 = nullptr, *cl_total = nullptr;
   double* cl_tp = nullptr;
   void* cl_sp = nullptr;
 };
 
-static int fill_params(const od_config* c, int n_pad, DevParams* P) {
+// Column offsets that can hold a pair within the cutoff, and their slab
+// reaches: ions m = max(|d| - 1, 0) columns apart are at least m w apart, so
+// an offset counts if 4 (mx^2 + my^2) < p2^2, and slabs dz apart if
+// 4 (mx^2 + my^2) q^2 + max(|dz| - 1, 0)^2 p2^2 < p2^2 q^2.  Returns the
+// number of forward offsets (off may be null).
+static int cell_offsets(CellGrid g, int* off) {
+  const int reach = (g.p2 + 1) / 2;
+  const int64_t p2 = g.p2, q = g.q;
+  int n = 0;
+  auto nbz = [&](int64_t M) {
+    int64_t j = 0;
+    while (4 * M * q * q + (j + 1) * (j + 1) * p2 * p2 < p2 * p2 * q * q) ++j;
+    return (int)j + 1;
+  };
+  for (int dy = 0; dy <= reach; ++dy)
+    for (int dx = dy ? -reach : 1; dx <= reach; ++dx) {
+      const int64_t mx = std::max(std::abs(dx) - 1, 0), my = std::max(dy - 1, 0), M = mx * mx + my * my;
+      if (4 * M >= p2 * p2) continue;
+      if (off && n < CC_MAX_FWD) off[n] = (dx & 255) | (dy & 255) << 8 | nbz(M) << 16;
+      ++n;
+    }
+  if (off && n <= CC_MAX_FWD) off[n] = nbz(0) << 16;
+  return n;
+}
+
+static int fill_params(const od_config* c, int n_pad, DevParams* P, CellGrid grid = CellGrid()) {
   std::memset(P, 0, sizeof(*P));
   const double L = 1.4426950408889634;
   P->n = c->n_ions;
@@ -348,15 +389,22 @@ static int fill_params(const od_config* c, int n_pad, DevParams* P) {
     P->rc32 = (float)(rc * L);
     P->rs32 = (float)(rs * L);
     P->invw32 = P->use_switch ? (float)(1.0 / ((rc - rs) * L)) : 0.0f;
-    P->col_w = c->cutoff / 4.0;
-    P->slab_h = c->cutoff / 16.0;
-    const double nxd = ceil(2.0 * c->R / P->col_w), nzd = ceil(c->H / P->slab_h);
     // sizes beyond the cell maximum are rejected by the caller (setup_cells)
-    const bool fits = nxd * nxd * nzd <= (double)OD_MAX_CELLS;
-    P->nx = fits ? (int)nxd : 1;
+    auto dims = [&](double w, double h, int* nx, int* nz) {
+      const double nxd = ceil(2.0 * c->R / w), nzd = ceil(c->H / h);
+      const bool fits = nxd * nxd * nzd <= (double)OD_MAX_CELLS;
+      *nx = fits ? (int)nxd : 1;
+      *nz = fits ? (int)nzd : 1;
+      return fits ? *nx * *nx * *nz : -1;
+    };
+    P->rc4_w = c->cutoff / 4.0;
+    P->rc4_h = c->cutoff / 16.0;
+    P->rc4_cells = dims(P->rc4_w, P->rc4_h, &P->rc4_nx, &P->rc4_nz);
+    P->col_w = 2.0 * c->cutoff / grid.p2;
+    P->slab_h = c->cutoff / grid.q;
+    P->n_cells = dims(P->col_w, P->slab_h, &P->nx, &P->nz);
     P->ny = P->nx;
-    P->nz = fits ? (int)nzd : 1;
-    P->n_cells = fits ? P->nx * P->ny * P->nz : -1;
+    P->n_fwd = cell_offsets(grid, P->off);
   }
   P->a32 = (float)(P->rho0 * L);
   P->linv32 = (float)(1.0 / L);
@@ -416,7 +464,7 @@ static void free_ctx(od_ctx* c) {
                   c->rowD, c->sym_sp, c->sym_acc, c->Gcut, c->scan_tsum, c->scan_toff, c->sc_tp, c->sc_sp, c->ckey[0], c->ckey[1], c->cval[0], c->cval[1], c->rs_hist,
                   c->rs_off, c->rs_total, c->cell_start, c->cell_chunks, c->item_off, c->items,
                   c->n_items, c->spos, c->tl.groups, c->tl.wg_group, c->tl.subs, c->tl.tp, c->tl.sp, c->cl_rng, c->cl_cnt,
-                  c->cl_u0, c->cl_total, c->cl_tp, c->cl_sp};
+                  c->cl_u0, c->cl_total, c->cl_tp, c->cl_sp, c->rc4_cell};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -688,47 +736,112 @@ static int sym_default_chunk(const std::vector<int>& be, int configured) {
   return ch;
 }
 
-// Units of k_cell_list for ions spread evenly over the cylinder: per group and
-// set the column's ions in the slab reach and the group's own length, in
-// 64-ion chunks, one more for the remainder.
-static double cell_list_units(const od_ctx* c, const od_config* cfg) {
+// Units of k_cell_list on a grid, for n ions spread evenly over the cylinder:
+// per group and set the column's ions in the slab reach and the group's own
+// length, in 64-ion chunks, and one for the remainder.
+static double cell_list_units(const od_config* cfg, int n, CellGrid g) {
   const double pi = 3.141592653589793;
-  const double w = cfg->cutoff / 4.0, h = cfg->cutoff / 16.0;
-  const double line = c->n / (pi * cfg->R * cfg->R * cfg->H) * w * w;  // ions per length of a column
+  const double w = 2.0 * cfg->cutoff / g.p2, h = cfg->cutoff / g.q;
+  const double line = n / (pi * cfg->R * cfg->R * cfg->H) * w * w;  // ions per length of a column
   const double len = std::min(cfg->H, CL_G / line);
+  int off[CC_MAX_FWD + 1];
+  const int n_fwd = cell_offsets(g, off);
   double per_group = 0.0;
-  for (int k = 0; k < CC_NSET; ++k) {
-    int dx = 0, dy = 0;
-    if (k < CC_NFWD) cc_fwd(k, dx, dy);
-    per_group += std::min(cfg->H, (2 * cc_nbz(dx, dy) + 1) * h + len) * line / 64.0 + 1.0;
+  for (int k = 0; k <= n_fwd; ++k)
+    per_group += std::min(cfg->H, (2 * (off[k] >> 16) + 1) * h + len) * line / 64.0 + 1.0;
+  const double nx = ceil(2.0 * cfg->R / w);
+  return ((double)n / CL_G + nx * nx) * per_group;
+}
+
+// Grid of the list.  Pairs out of range come from the columns' width and from
+// the length of a 64-ion chunk, so the best width follows the ion density
+// (and, in a narrow cylinder, how the columns fit it): the grid is the one of
+// least cost for ions spread evenly, in pair slots: for every 64 targets of a
+// column and every set, the sources in the window, half a chunk of padding,
+// and CELL_ENTRY_COST for the loads of its ranges.  Columns count by their
+// share inside the cylinder (4 x 4 points each; beyond 64 columns across, all
+// as full).  Force evaluation, columns cutoff/4 and slabs cutoff/16 -> this:
+// 130001 ions FP64 1.30 -> 0.47 ms (pair terms per in-range pair 15.9 ->
+// 5.4), FP32c 32768 ions 0.24 -> 0.06, 262144 1.07 -> 0.55, 2^20 5.6 -> 5.0;
+// at 2^22 the choice is columns of cutoff/4.
+constexpr double CELL_ENTRY_COST = 24.0;
+static CellGrid choose_grid(const od_config* cfg, int n) {
+  static const int qs[] = {8, 16, 32};
+  const double pi = 3.141592653589793;
+  const double dens = n / (pi * cfg->R * cfg->R * cfg->H);
+  CellGrid best;
+  double best_cost = 1e300;
+  for (int p2 = 1; p2 <= 10; ++p2) {
+    const double w = 2.0 * cfg->cutoff / p2, nxd = ceil(2.0 * cfg->R / w);
+    const bool bulk = nxd > 64.0;
+    const int nx = bulk ? 1 : (int)nxd;
+    std::vector<double> line(nx * nx);  // ions per length of a column
+    for (int i = 0; i < nx * nx; ++i) {
+      int in = bulk ? 16 : 0;
+      for (int s = 0; s < 16 && !bulk; ++s) {
+        const double x = (i % nx + (s % 4 + 0.5) / 4) * w - cfg->R, y = (i / nx + (s / 4 + 0.5) / 4) * w - cfg->R;
+        in += x * x + y * y < cfg->R * cfg->R;
+      }
+      line[i] = dens * w * w * in / 16.0;
+    }
+    for (int q : qs) {
+      const CellGrid g{p2, q};
+      int off[CC_MAX_FWD + 1];
+      const int n_fwd = cell_offsets(g, off);
+      const double h = cfg->cutoff / q;
+      if (n_fwd > CC_MAX_FWD || nxd * nxd * ceil(cfg->H / h) > std::max(65536.0, 0.5 * n)) continue;
+      double cost = 0.0;
+      for (int i = 0; i < nx * nx; ++i) {
+        if (line[i] == 0.0) continue;
+        const double len = std::min(cfg->H, 64.0 / line[i]);
+        const double chunks = line[i] * cfg->H / 64.0 + 0.5;
+        for (int k = 0; k <= n_fwd; ++k) {
+          const int x = i % nx + (int8_t)(off[k] & 255), y = i / nx + ((off[k] >> 8) & 255);
+          if (!bulk && (x < 0 || x >= nx || y >= nx)) continue;
+          const double lb = bulk ? line[0] : line[x + nx * y];
+          if (lb == 0.0) continue;
+          const double r = std::min(((off[k] >> 16) + 0.5) * h, cfg->H);
+          const double win = std::min(cfg->H, len + 2.0 * r - r * r / cfg->H);
+          cost += chunks * (k < n_fwd ? 1.0 : 0.5) * (win * lb + 32.0 + CELL_ENTRY_COST);
+        }
+      }
+      if (bulk) cost *= pi * cfg->R * cfg->R / (w * w);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = g;
+      }
+    }
   }
-  return ((double)c->n / CL_G + c->n_cols) * per_group;
+  return best;
 }
 
 // Whether the context runs k_cell_list: where its partials, at twice the even
-// spread's units, fit CELL_LIST_MAX_BYTES; in FP32c only where the column
-// kernel's waves (one per column and set, at most) are too few to fill the
-// chip, and not if the configuration fixes a variant of that kernel.  Force
-// evaluation, column kernel -> list: 131072 ions in 64 columns 5.37 -> 1.81
-// ms, 16384 0.38 -> 0.23; with 1600 columns 32768 ions 0.21 -> 0.24, 2^20 5.51
-// -> 5.61, 2^22 53.2 -> 52.6.
+// spread's units, fit CELL_LIST_MAX_BYTES, unless the configuration fixes a
+// variant of k_pair32_symcol.
 constexpr double CELL_LIST_MAX_BYTES = 24e9;
-constexpr int CELL_COLUMN_WAVES = 16384;
-static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, int* cap) {
-  const double units = 2.0 * cell_list_units(c, cfg) + 4096.0;
+static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, CellGrid g, int* cap) {
+  const double units = 2.0 * cell_list_units(cfg, c->n, g) + 4096.0;
   const bool fp32 = c->prec == OD_PREC_FP32C;
   *cap = (int)std::min(units, 1e9);
-  if (fp32 && (cfg->sym_tile > 0 || c->n_cols * CC_NSET >= CELL_COLUMN_WAVES)) return false;
+  if (fp32 && cfg->sym_tile > 0) return false;
   return units * 192.0 * (fp32 ? 4.0 : 8.0) <= CELL_LIST_MAX_BYTES;
 }
 
-static int setup_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
+// hp: the parameters with od_get_cells' grid; gets the context's own
+static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
   c->cut = 0;
   if (!(cfg->cutoff > 0.0)) return OD_OK;
-  if (hp.n_cells < 0)
+  if (hp.rc4_cells < 0)
     return set_err(OD_ERR_ARG, "cutoff %g nm in a cylinder R = %g, H = %g nm gives more than %d cells", cfg->cutoff,
                    cfg->R, cfg->H, OD_MAX_CELLS);
   c->cut = 1;
+  const CellGrid g = choose_grid(cfg, c->n);
+  c->list = cell_list_chosen(c, cfg, g, &c->cl_cap) ? 1 : 0;
+  if (c->list) {
+    c->grid = g;
+    fill_params(cfg, c->n_pad, &hp, g);
+  }
+  c->n_set = hp.n_fwd + 1;
   c->n_cells = hp.n_cells;
   c->n_cols = hp.nx * hp.ny;
   c->nx = hp.nx;
@@ -738,10 +851,9 @@ static int setup_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   c->rs_passes = 1;
   while (c->rs_passes < 4 && ((uint64_t)c->n_cells >> (8 * c->rs_passes)) != 0) ++c->rs_passes;
   c->rs_nblk = (c->n_pad + RS_ITEMS - 1) / RS_ITEMS;
-  c->list = cell_list_chosen(c, cfg, &c->cl_cap) ? 1 : 0;
   c->item_len = c->list ? CL_G : 64;
   c->max_items = c->n_pad / c->item_len + c->n_cols + 1;
-  c->n_entries = c->list ? c->max_items * CC_NSET : 0;
+  c->n_entries = c->list ? c->max_items * c->n_set : 0;
   const size_t np = c->n_pad;
   int rc = OD_OK;
   if ((rc = dalloc(&c->ckey[0], np * 4)) || (rc = dalloc(&c->ckey[1], np * 4)) || (rc = dalloc(&c->cval[0], np * 4)) ||
@@ -762,14 +874,14 @@ static int setup_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   if (c->list) {
     const size_t ne = (size_t)c->n_entries + 1;
     if ((rc = dalloc(&c->cl_rng, ne * sizeof(int2))) || (rc = dalloc(&c->cl_cnt, ne * 4)) ||
-        (rc = dalloc(&c->cl_u0, ne * 4)) || (rc = dalloc(&c->cl_total, 4)) ||
+        (rc = dalloc(&c->cl_u0, ne * 4)) || (rc = dalloc(&c->rc4_cell, np * 4)) || (rc = dalloc(&c->cl_total, 4)) ||
         (rc = dalloc(&c->cl_tp, ((size_t)CL_WAVES + c->max_items) * 3 * CL_G * 8)) ||
         (rc = dalloc(&c->cl_sp, (size_t)c->cl_cap * 192 * (c->prec == OD_PREC_FP32C ? 4 : 8))))
       return rc;
   }
   if (c->prec == OD_PREC_FP32C) {
-    if ((rc = dalloc(&c->sc_tp, (size_t)CC_NSET * 3 * np * 8)) ||
-        (rc = dalloc(&c->sc_sp, (size_t)CC_NSET * 3 * np * 4)))
+    if ((rc = dalloc(&c->sc_tp, (size_t)c->n_set * 3 * np * 8)) ||
+        (rc = dalloc(&c->sc_sp, (size_t)c->n_set * 3 * np * 4)))
       return rc;
     c->sc_var = cell_variant_of(cfg->sym_tile);
     if (c->sc_var < 0) return set_err(OD_ERR_ARG, "cutoff mode: sym_tile %d outside [0, %d]", cfg->sym_tile, CC_N_VARIANTS);
@@ -1046,7 +1158,8 @@ template <class T>
 static int build_cells_t(od_ctx* c, const double* X, const uint32_t* flags, const void* pos) {
   using PV = typename Pos<T>::V;
   const int np = c->n_pad, nb = c->nb, nc = c->n_cells;
-  hipLaunchKernelGGL(k_bin, dim3(nb), dim3(256), 0, c->stream, c->dP, X, flags, c->ckey[0], c->cval[0]);
+  hipLaunchKernelGGL(k_bin, dim3(nb), dim3(256), 0, c->stream, c->dP, X, flags, c->ckey[0], c->cval[0],
+                     c->rc4_cell);
   for (int pass = 0; pass < c->rs_passes; ++pass) {
     const int in = pass & 1, out = 1 - in, shift = 8 * pass;
     hipLaunchKernelGGL(k_rs_hist, dim3(c->rs_nblk), dim3(256), 0, c->stream, c->ckey[in], np, shift, c->rs_nblk,
@@ -1102,7 +1215,7 @@ static int launch_forces_t(od_ctx* c, const double* X, const void* pos, const ui
   if constexpr (std::is_same<T, float>::value) {
     // symmetric: forward neighbour columns and the own column, per-ion reduction
     const float4* sp4 = (const float4*)c->spos;
-    const dim3 g(c->n_cols * CC_NSET);
+    const dim3 g(c->n_cols * c->n_set);
     const int ki = c->sc_var * 2 + (sw ? 1 : 0);
     hipLaunchKernelGGL(cell_sym_kernels[ki], g, dim3(64), 0, c->stream, c->dP, sp4, c->skey, c->cell_start, n_units,
                        c->cl_cap, c->sc_tp, c->sc_sp);
@@ -1272,7 +1385,7 @@ extern "C" int od_update_config(od_ctx* c, const od_config* cfg) {
                    "cylinder must stay the same");
   HIPCHK(hipSetDevice(c->dev));
   DevParams hp;
-  CHKRET(fill_params(cfg, c->n_pad, &hp));
+  CHKRET(fill_params(cfg, c->n_pad, &hp, c->grid));
   HIPCHK(hipStreamSynchronize(c->stream));
   HIPCHK(hipMemcpy(c->dP, &hp, sizeof(hp), hipMemcpyHostToDevice));
   const int keep_chunk = c->cfg.sym_chunk, keep_tile = c->cfg.sym_tile;
@@ -1412,25 +1525,37 @@ extern "C" int od_get_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sorted_ion
   if (!c->cut) return set_err(OD_ERR_STATE, "od_get_cells: context has no cutoff (no cell list)");
   HIPCHK(hipSetDevice(c->dev));
   std::vector<uint32_t> key(c->n_pad), val(c->n_pad);
-  HIPCHK(hipMemcpyAsync(key.data(), c->skey, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(val.data(), c->sval, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  DevParams hp;
+  fill_params(&c->cfg, c->n_pad, &hp);
+  const uint32_t n_cells = (uint32_t)hp.rc4_cells;
+  if (c->rc4_cell) {
+    // the forces' grid is another: (cell, ion) order of the binned ions
+    HIPCHK(hipMemcpyAsync(key.data(), c->rc4_cell, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    for (int i = 0; i < c->n_pad; ++i) val[i] = (uint32_t)i;
+    std::stable_sort(val.begin(), val.end(), [&](uint32_t a, uint32_t b) { return key[a] < key[b]; });
+    std::vector<uint32_t> sorted(c->n_pad);
+    for (int p = 0; p < c->n_pad; ++p) sorted[p] = std::min(key[val[p]], n_cells);
+    key.swap(sorted);
+  } else {
+    HIPCHK(hipMemcpyAsync(key.data(), c->skey, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(val.data(), c->sval, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+  }
   int64_t nb = 0;
   for (int p = 0; p < c->n_pad; ++p) {
     const uint32_t i = val[p];
     if ((int)i < c->n && cell_of_ion) cell_of_ion[i] = (int32_t)key[p];
-    if ((int)key[p] < c->n_cells) {
+    if (key[p] < n_cells) {
       if (sorted_ions) sorted_ions[nb] = (int32_t)i;
       ++nb;
     }
   }
   if (n_binned) *n_binned = nb;
   if (dims) {
-    DevParams hp;
-    fill_params(&c->cfg, c->n_pad, &hp);
-    dims[0] = hp.nx;
-    dims[1] = hp.ny;
-    dims[2] = hp.nz;
+    dims[0] = hp.rc4_nx;
+    dims[1] = hp.rc4_nx;
+    dims[2] = hp.rc4_nz;
   }
   return OD_OK;
 }
@@ -1442,6 +1567,8 @@ extern "C" int od_get_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sorted_ion
 // ordered terms (force and reaction), its own-group tiles one.
 static int64_t cell_candidates(const od_ctx* c, const std::vector<int>& cs, const std::vector<uint32_t>& key) {
   const int nx = c->nx, ny = c->ny, nz = c->nz;
+  DevParams hp;
+  fill_params(&c->cfg, c->n_pad, &hp, c->grid);
   auto range = [&](int bx, int by, int blo, int bhi, int nbz, int64_t& s0, int64_t& s1) {
     s0 = s1 = 0;
     if (bx < 0 || bx >= nx || by < 0 || by >= ny) return;
@@ -1460,15 +1587,14 @@ static int64_t cell_candidates(const od_ctx* c, const std::vector<int>& cs, cons
       const int MTv = cell_variant_mt[c->sc_var];
       const bool split = cell_variant_split[c->sc_var];
       const int G = 64 * MTv;
-      for (int k = 0; k < CC_NSET; ++k) {
-        const bool own = k == CC_NFWD;
-        int dx = 0, dy = 0;
-        if (!own) cc_fwd(k, dx, dy);
+      for (int k = 0; k < c->n_set; ++k) {
+        const bool own = k == c->n_set - 1;
+        int dx, dy, nbz;
+        cc_off(hp, k, dx, dy, nbz);
         const int bx = ax + dx, by = ay + dy;
         if (bx < 0 || bx >= nx || by >= ny) continue;
         const int cb = nz * (bx + nx * by);
         if (!own && cs[cb] == cs[cb + nz]) continue;
-        const int nbz = cc_nbz(dx, dy);
         for (int t0 = a0; t0 < a1; t0 += G) {
           const int t1 = std::min(t0 + G, a1);
           const int blo = (int)key[t0] - cA, bhi = (int)key[t1 - 1] - cA;
@@ -1502,11 +1628,11 @@ static int64_t cell_candidates(const od_ctx* c, const std::vector<int>& cs, cons
       for (int t0 = a0; t0 < a1; t0 += 64) {
         const int tl = std::min(t0 + 63, a1 - 1);
         const int blo = (int)key[t0] - cA, bhi = (int)key[tl] - cA;
-        for (int k = 0; k < CC_NOFF; ++k) {
-          int dx, dy;
-          cc_off(k, dx, dy);
+        for (int k = 0; k < 2 * c->n_set - 1; ++k) {
+          int dx, dy, nbz;
+          cc_off(hp, k, dx, dy, nbz);
           int64_t s0, s1;
-          range(ax + dx, ay + dy, blo, bhi, cc_nbz(dx, dy), s0, s1);
+          range(ax + dx, ay + dy, blo, bhi, nbz, s0, s1);
           total += 64 * (s1 - s0);
         }
       }
@@ -1844,11 +1970,9 @@ static int tune_cells(od_ctx* c, int reps, int* chosen_var) {
   CHKRET(dalloc(&Fs, (size_t)3 * c->n_pad * 8));
   int rc = load_positions(c, c->X, c->pi, c->pj);
   double best_ms = 1e300;
-  const int had_list = c->list;
-  int best = had_list ? -1 : c->sc_var;
-  for (int v = had_list ? -1 : 0; v < CC_N_VARIANTS && rc == OD_OK; ++v) {
-    c->list = v < 0 ? 1 : 0;
-    c->sc_var = v < 0 ? CC_DEFAULT : v;
+  int best = c->sc_var;
+  for (int v = 0; v < CC_N_VARIANTS && rc == OD_OK; ++v) {
+    c->sc_var = v;
     rc = launch_forces(c, c->X, c->pj, nullptr, Fs, false);  // warm-up
     if (rc == OD_OK && hipEventRecord(c->ev0, c->stream) != hipSuccess) rc = set_err(OD_ERR_HIP, "hipEventRecord");
     for (int r = 0; r < reps && rc == OD_OK; ++r) rc = launch_forces(c, c->X, c->pj, nullptr, Fs, false);
@@ -1862,8 +1986,7 @@ static int tune_cells(od_ctx* c, int reps, int* chosen_var) {
     }
   }
   (void)hipFree(Fs);
-  c->list = best < 0 ? 1 : 0;
-  c->sc_var = best < 0 ? CC_DEFAULT : best;
+  c->sc_var = best;
   *chosen_var = best;
   return rc;
 }
@@ -1872,7 +1995,7 @@ extern "C" int od_tune(od_ctx* c, int32_t reps, int32_t* sym_chunk, int32_t* sym
   if (!c) return set_err(OD_ERR_ARG, "null context");
   if (reps < 1 || reps > 100) return set_err(OD_ERR_ARG, "reps %d outside [1, 100]", reps);
   int chosen = 0, var = -1;
-  if (c->cut && c->prec == OD_PREC_FP32C) {
+  if (c->cut && c->prec == OD_PREC_FP32C && !c->list) {
     if (!c->have_ions) return set_err(OD_ERR_STATE, "od_tune needs the ions (call od_set_ions first)");
     HIPCHK(hipSetDevice(c->dev));
     CHKRET(tune_cells(c, reps, &var));
