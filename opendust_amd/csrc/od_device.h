@@ -226,9 +226,9 @@ __device__ __forceinline__ void pair32_cut(float xi, float yi, float zi, float x
   az = __builtin_fmaf(h, dz, az);
 }
 
-// the truncated FP64 law's h, by selection (no branch)
+// the FP64 law's h inside the cutoff (SW: switched)
 template <bool SW>
-__device__ __forceinline__ double pair64_cut_h(double r2, double rho0, double rc, double rs, double invw) {
+__device__ __forceinline__ double pair64_cut_h(double r2, double rho0, double rs, double invw) {
   const double y = rsqrt64(r2);
   const double r = r2 * y;
   const double e = exp_neg64(r);
@@ -241,7 +241,7 @@ __device__ __forceinline__ double pair64_cut_h(double r2, double rho0, double rc
     const double S = fma(x2 * x, fma(x, fma(x, -6.0, 15.0), -10.0), 1.0);
     h = fma(h, S, e * yz * (30.0 * x2 * omx * omx * invw));
   }
-  return (r < rc) ? h : 0.0;
+  return h;
 }
 
 __device__ __forceinline__ void pair64_cut(double xi, double yi, double zi, double xj, double yj, double zj,

@@ -95,7 +95,7 @@ struct DevParams {
   double rho0;
   // truncation (cutoff mode): FP32 values in L/lambda units, FP64 in lambda units
   int use_cut, use_switch;
-  float rc32, rs32, invw32;
+  float rc32, rs32, invw32, rc2_32;
   double rc64, rs64, invw64;
   // cell grid (nm): columns of col_w in x and y, slabs of slab_h in z
   double col_w, slab_h;
@@ -387,6 +387,7 @@ static int fill_params(const od_config* c, int n_pad, DevParams* P, CellGrid gri
     P->rs64 = rs;
     P->invw64 = P->use_switch ? 1.0 / (rc - rs) : 0.0;
     P->rc32 = (float)(rc * L);
+    P->rc2_32 = (float)(rc * L * rc * L);
     P->rs32 = (float)(rs * L);
     P->invw32 = P->use_switch ? (float)(1.0 / ((rc - rs) * L)) : 0.0f;
     // sizes beyond the cell maximum are rejected by the caller (setup_cells)
