@@ -212,6 +212,24 @@ __device__ double block_sum256(double v, double* lds) {
   return r;
 }
 
+// N sums at once over a 256-thread block, each in block_sum256's order: thread k
+// < N returns sum k.  Two calls in a row need two lds arrays (the first call's
+// readers may still be at it).
+template <int N>
+__device__ __forceinline__ double block_sums256(double (&v)[N], double (*lds)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < N; ++k) lds[wave][k] = v[k];
+  __syncthreads();
+  const int k = min((int)threadIdx.x, N - 1);
+  return (lds[0][k] + lds[1][k]) + (lds[2][k] + lds[3][k]);
+}
+
 // ---------------------------------------------------------------------------
 // positions -> kernel coordinates
 // ---------------------------------------------------------------------------
@@ -227,8 +245,8 @@ __global__ __launch_bounds__(256) void k_load_pos(const double* __restrict__ X, 
 }
 
 #include "od_kernels_pair.inc"
-#include "od_kernels_tile.inc"
 #include "od_kernels_step.inc"
+#include "od_kernels_tile.inc"
 #include "od_kernels_trap.inc"
 #include "od_kernels_cell.inc"
 
@@ -293,6 +311,7 @@ struct od_ctx {
   std::vector<int> band_row, band_slot;
   // wave tiles (k_pair_tile)
   int tile = 0;
+  bool with_rows = false;  // launch_pair: the absorbed ions' rows ride on the reduction
   TilePlan tl;
   // cutoff mode: cell list; Gcut: flagged sources' share of the drift-state force;
   // sc_tp, sc_sp: partials of the symmetric cell kernel (FP32c)
@@ -541,9 +560,19 @@ static void launch_tile(const TilePlan& t, hipStream_t st, const DevParams* dP, 
 }
 
 template <class T>
-static void launch_tile_reduce(const TilePlan& t, hipStream_t st, const DevParams* dP, int stride, double* F) {
-  hipLaunchKernelGGL(k_tile_reduce<T>, dim3(t.n_sub), dim3(256), 0, st, dP, (const TileGroup*)t.groups,
-                     (const int4*)t.subs, t.per, t.mt * t.nw, (const double*)t.tp, (const T*)t.sp, stride, F);
+static void launch_tile_reduce(const TilePlan& t, hipStream_t st, const DevParams* dP, int stride, double* F,
+                               const AbsorbedRows<T>& ab) {
+  hipLaunchKernelGGL(k_tile_reduce<T>, dim3(t.n_sub + ab.n), dim3(256), 0, st, dP, 0, t.n_sub,
+                     (const TileGroup*)t.groups, (const int4*)t.subs, t.per, t.mt * t.nw, (const double*)t.tp,
+                     (const T*)t.sp, stride, F, ab);
+}
+
+// the absorbed ions' rows alone (see k_tile_reduce)
+template <class T>
+static void launch_absorbed_rows(const TilePlan& t, hipStream_t st, const DevParams* dP, const AbsorbedRows<T>& ab) {
+  hipLaunchKernelGGL(k_tile_reduce<T>, dim3(ab.n), dim3(256), 0, st, dP, t.n_sub, t.n_sub, (const TileGroup*)t.groups,
+                     (const int4*)t.subs, t.per, t.mt * t.nw, (const double*)t.tp, (const T*)t.sp, 0,
+                     (double*)nullptr, ab);
 }
 
 // launch geometry of the pair kernel
@@ -1067,6 +1096,14 @@ static void mark(od_ctx* c, int stage) {
   c->kst[c->kn++] = stage;
 }
 
+constexpr int ABSORBED_ROWS = 64;  // blocks for the absorbed ions' rows
+template <class T>
+static AbsorbedRows<T> absorbed_rows(const od_ctx* c, int n) {
+  using PV = typename Pos<T>::V;
+  return {n, (1u << c->cfg.n_dust) - 1u, nullptr, (const PV*)c->pi, (const PV*)c->list_old, c->n_flag, c->list_ion,
+          c->flags, c->rowD};
+}
+
 // Pair force of sources pj on targets pi into F, optionally timed.  The
 // symmetric kernel treats one array as both targets and sources: it is only
 // used when pi == pj.
@@ -1080,10 +1117,11 @@ static int launch_pair(od_ctx* c, const void* pi, const void* pj, double* F, boo
     else
       launch_tile<double>(c->tl, c->stream, c->dP, pj);
     if (timed) HIPCHK(hipEventRecord(c->ev1, c->stream));
+    const int rows = c->with_rows ? ABSORBED_ROWS : 0;
     if (c->prec == OD_PREC_FP32C)
-      launch_tile_reduce<float>(c->tl, c->stream, c->dP, c->n_pad, F);
+      launch_tile_reduce<float>(c->tl, c->stream, c->dP, c->n_pad, F, absorbed_rows<float>(c, rows));
     else
-      launch_tile_reduce<double>(c->tl, c->stream, c->dP, c->n_pad, F);
+      launch_tile_reduce<double>(c->tl, c->stream, c->dP, c->n_pad, F, absorbed_rows<double>(c, rows));
     return OD_OK;
   }
   if (c->sym && pi == pj) {
@@ -1257,15 +1295,27 @@ static int launch_step_t(od_ctx* c, bool timed) {
   hipLaunchKernelGGL(k_kick_drift<T>, dim3(nb), dim3(256), 0, c->stream, c->dP, (const int*)nullptr, c->X, c->V,
                      c->F, c->q, c->st, (PV*)c->pi, (PV*)c->pj, c->flags, c->block_cnt, c->err);
   mark(c, OD_STAGE_LIST);
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->stream, c->block_cnt, nb, c->block_off, c->n_flag);
-  hipLaunchKernelGGL(k_list<T>, dim3(nb), dim3(256), 0, c->stream, c->flags, c->block_cnt, c->block_off, c->n,
-                     (const PV*)c->pi, c->slot_of, c->list_ion, (PV*)c->list_old);
+  const bool few = nb <= FEW_BLOCKS;
+  if (few) {
+    hipLaunchKernelGGL(k_scan_list<T>, dim3(nb), dim3(256), 0, c->stream, c->flags, c->block_cnt, c->block_off,
+                       c->n_flag, c->n, (const PV*)c->pi, c->slot_of, c->list_ion, (PV*)c->list_old);
+  } else {
+    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->stream, c->block_cnt, nb, c->block_off, c->n_flag);
+    hipLaunchKernelGGL(k_list<T>, dim3(nb), dim3(256), 0, c->stream, c->flags, c->block_cnt, c->block_off, c->n,
+                       (const PV*)c->pi, c->slot_of, c->list_ion, (PV*)c->list_old);
+  }
   // flagged ions are parked in pj, as sources and as targets (cutoff mode:
   // left out of the cell list)
-  CHKRET(launch_forces_t<T>(c, c->X, c->pj, c->flags, c->F, timed));
   const uint32_t dust_bits = (c->cfg.n_dust > 0) ? ((1u << c->cfg.n_dust) - 1u) : 0u;
+  const bool ride = c->tile && few && dust_bits;
+  c->with_rows = ride && !c->kprof;
+  const int rc = launch_forces_t<T>(c, c->X, c->pj, c->flags, c->F, timed);
+  c->with_rows = false;
+  CHKRET(rc);
   mark(c, OD_STAGE_ROWS_ABSORBED);
-  if (dust_bits) {
+  if (ride) {
+    if (c->kprof) launch_absorbed_rows<T>(c->tl, c->stream, c->dP, absorbed_rows<T>(c, ABSORBED_ROWS));
+  } else if (dust_bits) {
     if (c->cut)
       hipLaunchKernelGGL(k_rows_cell<T>, dim3(c->rows_grid), dim3(256), 0, c->stream, c->dP, c->X,
                          (const PV*)c->spos, c->cell_start, c->n_flag, (const PV*)c->list_old,
@@ -1285,6 +1335,25 @@ static int launch_step_t(od_ctx* c, bool timed) {
                      (const PV*)c->pi, (PV*)c->pj, c->flags, c->n_flag, c->slot_of, (const PV*)c->list_old,
                      (PV*)c->list_new, c->face, c->rowD, c->cut ? (const double*)c->Gcut : (const double*)nullptr,
                      c->partials);
+  if (few && !c->cut) {
+    // one launch; one per part when the stages are timed
+    auto part = [&](int stage, int first, int blocks) {
+      mark(c, stage);
+      hipLaunchKernelGGL(k_step_end<T>, dim3(blocks), dim3(256), 0, c->stream, c->dP, (const int*)nullptr, first, 1,
+                         END_ROWS, c->block_off, nb, c->F, (const PV*)c->pj, c->flags, c->n_flag,
+                         (const PV*)c->list_new, c->list_ion, (const double*)c->partials, c->q, c->st, c->rec,
+                         std::max(1, c->cfg.n_dust), 1);
+    };
+    if (c->kprof) {
+      part(OD_STAGE_ROWS_REINJECTED, 1, END_ROWS);
+      part(OD_STAGE_INFLOW, 1 + END_ROWS, nb);
+      part(OD_STAGE_DUST, 0, 1);
+    } else {
+      part(OD_STAGE_DUST, 0, 1 + END_ROWS + nb);
+    }
+    mark(c, -1);
+    return OD_OK;
+  }
   mark(c, OD_STAGE_ROWS_REINJECTED);
   if (c->cut)
     hipLaunchKernelGGL(k_rows_cell<T>, dim3(c->rows_grid), dim3(256), 0, c->stream, c->dP, c->X, (const PV*)c->spos,
