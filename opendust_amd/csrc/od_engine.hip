@@ -244,6 +244,19 @@ __global__ __launch_bounds__(256) void k_load_pos(const double* __restrict__ X, 
   pj[i] = p;
 }
 
+// host layout [n][3] <-> the engine's three arrays of n, `stride` apart
+__global__ __launch_bounds__(256) void k_pack3(const double* __restrict__ s, int n, int stride,
+                                               double* __restrict__ a) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t < 3 * (int64_t)n) a[t] = s[(t % 3) * stride + t / 3];
+}
+
+__global__ __launch_bounds__(256) void k_unpack3(const double* __restrict__ a, int n, int stride,
+                                                 double* __restrict__ s) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t < 3 * (int64_t)n) s[(t % 3) * stride + t / 3] = a[t];
+}
+
 #include "od_kernels_pair.inc"
 #include "od_kernels_step.inc"
 #include "od_kernels_tile.inc"
@@ -1406,11 +1419,12 @@ extern "C" int od_set_ions(od_ctx* c, const double* x, const double* v, int64_t 
     if (!std::isfinite(x[i]) || !std::isfinite(v[i]))
       return set_err(OD_ERR_NONFINITE, "od_set_ions: non-finite value at ion %lld", (long long)(i / 3));
   HIPCHK(hipSetDevice(c->dev));
-  std::vector<double> sx, sv;
-  aos_to_soa(x, c->n, c->n_pad, sx);
-  aos_to_soa(v, c->n, c->n_pad, sv);
-  HIPCHK(hipMemcpyAsync(c->X, sx.data(), sx.size() * 8, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(c->V, sv.data(), sv.size() * 8, hipMemcpyHostToDevice, c->stream));
+  // rowF and rowD hold nothing between steps
+  const dim3 g((unsigned)((3 * n + 255) / 256));
+  HIPCHK(hipMemcpyAsync(c->rowF, x, 3 * n * 8, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(hipMemcpyAsync(c->rowD, v, 3 * n * 8, hipMemcpyHostToDevice, c->stream));
+  hipLaunchKernelGGL(k_unpack3, g, dim3(256), 0, c->stream, (const double*)c->rowF, (int)n, c->n_pad, c->X);
+  hipLaunchKernelGGL(k_unpack3, g, dim3(256), 0, c->stream, (const double*)c->rowD, (int)n, c->n_pad, c->V);
   CHKRET(load_positions(c, c->X, c->pi, c->pj));
   CHKRET(launch_forces(c, c->X, c->pj, nullptr, c->F, false));
   HIPCHK(hipGetLastError());
@@ -1422,19 +1436,16 @@ extern "C" int od_set_ions(od_ctx* c, const double* x, const double* v, int64_t 
 extern "C" int od_get_ions(od_ctx* c, double* x, double* v) {
   if (!c) return set_err(OD_ERR_ARG, "null context");
   HIPCHK(hipSetDevice(c->dev));
-  std::vector<double> s(3 * (size_t)c->n_pad);
-  if (x) {
-    HIPCHK(hipMemcpyAsync(s.data(), c->X, s.size() * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    for (int i = 0; i < c->n; ++i)
-      for (int k = 0; k < 3; ++k) x[3 * (size_t)i + k] = s[(size_t)k * c->n_pad + i];
-  }
-  if (v) {
-    HIPCHK(hipMemcpyAsync(s.data(), c->V, s.size() * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    for (int i = 0; i < c->n; ++i)
-      for (int k = 0; k < 3; ++k) v[3 * (size_t)i + k] = s[(size_t)k * c->n_pad + i];
-  }
+  double* dst[2] = {x, v};
+  const double* src[2] = {c->X, c->V};
+  double* tmp[2] = {c->rowF, c->rowD};  // hold nothing between steps
+  const dim3 g((unsigned)((3 * (size_t)c->n + 255) / 256));
+  for (int k = 0; k < 2; ++k)
+    if (dst[k]) hipLaunchKernelGGL(k_pack3, g, dim3(256), 0, c->stream, src[k], c->n, c->n_pad, tmp[k]);
+  HIPCHK(hipGetLastError());
+  for (int k = 0; k < 2; ++k)
+    if (dst[k]) HIPCHK(hipMemcpyAsync(dst[k], tmp[k], 3 * (size_t)c->n * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
   return OD_OK;
 }
 
