@@ -496,8 +496,7 @@ static void free_ctx(od_ctx* c) {
                   c->slot_of, c->list_ion, c->err, c->rec, c->wg_tab, c->wg_base, c->sym_tp, c->sym_dg,
                   c->rowD, c->sym_sp, c->sym_acc, c->Gcut, c->scan_tsum, c->scan_toff, c->sc_tp, c->sc_sp, c->ckey[0], c->ckey[1], c->cval[0], c->cval[1], c->rs_hist,
                   c->rs_off, c->rs_total, c->cell_start, c->cell_chunks, c->item_off, c->items,
-                  c->n_items, c->spos, c->tl.groups, c->tl.wg_group, c->tl.subs, c->tl.tp, c->tl.sp, c->cl_rng, c->cl_cnt,
-                  c->cl_u0, c->cl_total, c->cl_tp, c->cl_sp, c->rc4_cell};
+                  c->n_items, c->spos, c->tl.subs, c->tl.tp, c->cl_rng, c->cl_tp, c->rc4_cell};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -515,11 +514,8 @@ static int dalloc(P** p, size_t bytes) {
   return OD_OK;
 }
 
-// (Re)builds the wave-tile plan *t; its old buffers are freed first.
+// Builds the wave-tile plan *t (once per context).
 static int tile_build(TilePlan* t, const TileSims& sims, bool fp32) {
-  void* old[] = {t->groups, t->wg_group, t->subs, t->tp, t->sp};
-  for (void* q : old)
-    if (q) (void)hipFree(q);
   *t = TilePlan();
   tile_shape(sims, fp32, &t->mt, &t->nw);
   const int gm = t->mt * t->nw;
@@ -548,14 +544,23 @@ static int tile_build(TilePlan* t, const TileSims& sims, bool fp32) {
     wg[b] = g;
   }
   const size_t segs = (size_t)t->n_wg + t->n_groups;
-  int rc = OD_OK;
-  if ((rc = dalloc(&t->groups, groups.size() * sizeof(TileGroup))) || (rc = dalloc(&t->wg_group, wg.size() * 4)) ||
-      (rc = dalloc(&t->subs, subs.size() * sizeof(int4))) || (rc = dalloc(&t->tp, segs * 192 * gm * 8)) ||
-      (rc = dalloc(&t->sp, (size_t)u * 192 * (fp32 ? 4 : 8))))
-    return rc;
-  HIPCHK(hipMemcpy(t->groups, groups.data(), groups.size() * sizeof(TileGroup), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(t->wg_group, wg.data(), wg.size() * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(t->subs, subs.data(), subs.size() * sizeof(int4), hipMemcpyHostToDevice));
+  // one allocation and one upload for the tables, one for the partial sums
+  // (each call costs a new context some tens of microseconds)
+  const size_t b_sub = subs.size() * sizeof(int4), b_grp = groups.size() * sizeof(TileGroup), b_wg = wg.size() * 4;
+  std::vector<char> tab(b_sub + b_grp + b_wg);
+  std::memcpy(tab.data(), subs.data(), b_sub);
+  std::memcpy(tab.data() + b_sub, groups.data(), b_grp);
+  std::memcpy(tab.data() + b_sub + b_grp, wg.data(), b_wg);
+  char *d_tab = nullptr, *d_sum = nullptr;
+  const size_t b_tp = segs * 192 * gm * 8;
+  CHKRET(dalloc(&d_tab, tab.size()));
+  t->subs = (int4*)d_tab;
+  t->groups = (TileGroup*)(d_tab + b_sub);
+  t->wg_group = (int*)(d_tab + b_sub + b_grp);
+  CHKRET(dalloc(&d_sum, b_tp + (size_t)u * 192 * (fp32 ? 4 : 8)));
+  t->tp = (double*)d_sum;
+  t->sp = d_sum + b_tp;
+  HIPCHK(hipMemcpy(d_tab, tab.data(), tab.size(), hipMemcpyHostToDevice));
   return OD_OK;
 }
 
@@ -915,12 +920,16 @@ static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
   if ((rc = dalloc(&c->scan_tsum, n_tiles * 4)) || (rc = dalloc(&c->scan_toff, n_tiles * 4))) return rc;
   c->sc_var = CC_DEFAULT;
   if (c->list) {
+    // one allocation for the tables, one for the partial sums
     const size_t ne = (size_t)c->n_entries + 1;
-    if ((rc = dalloc(&c->cl_rng, ne * sizeof(int2))) || (rc = dalloc(&c->cl_cnt, ne * 4)) ||
-        (rc = dalloc(&c->cl_u0, ne * 4)) || (rc = dalloc(&c->rc4_cell, np * 4)) || (rc = dalloc(&c->cl_total, 4)) ||
-        (rc = dalloc(&c->cl_tp, ((size_t)CL_WAVES + c->max_items) * 3 * CL_G * 8)) ||
-        (rc = dalloc(&c->cl_sp, (size_t)c->cl_cap * 192 * (c->prec == OD_PREC_FP32C ? 4 : 8))))
+    const size_t b_tp = ((size_t)CL_WAVES + c->max_items) * 3 * CL_G * 8;
+    if ((rc = dalloc(&c->cl_rng, ne * 16 + 4)) || (rc = dalloc(&c->rc4_cell, np * 4)) ||
+        (rc = dalloc(&c->cl_tp, b_tp + (size_t)c->cl_cap * 192 * (c->prec == OD_PREC_FP32C ? 4 : 8))))
       return rc;
+    c->cl_cnt = (int*)(c->cl_rng + ne);
+    c->cl_u0 = c->cl_cnt + ne;
+    c->cl_total = c->cl_u0 + ne;
+    c->cl_sp = (char*)c->cl_tp + b_tp;
   }
   if (c->prec == OD_PREC_FP32C) {
     if ((rc = dalloc(&c->sc_tp, (size_t)c->n_set * 3 * np * 8)) ||
@@ -1068,7 +1077,6 @@ extern "C" int od_create(const od_config* cfg, od_ctx** out) {
   const size_t np = c->n_pad;
   if ((rc = dalloc(&c->dP, sizeof(DevParams))) || (rc = dalloc(&c->X, 3 * np * 8)) ||
       (rc = dalloc(&c->V, 3 * np * 8)) || (rc = dalloc(&c->F, 3 * np * 8)) ||
-      (rc = dalloc(&c->Fpart, (c->n_chunks > 1 ? c->n_chunks : 1) * 3 * np * 8)) ||
       (rc = dalloc(&c->q, OD_MAX_DUST * 8)) || (rc = dalloc(&c->partials, (size_t)c->nb * OD_MAX_DUST * 8 * 8)) ||
       (rc = dalloc(&c->rowF, 3 * np * 8)) || (rc = dalloc(&c->pi, np * c->pos_bytes)) ||
       (rc = dalloc(&c->pj, np * c->pos_bytes)) || (rc = dalloc(&c->list_old, np * c->pos_bytes)) ||
@@ -1078,6 +1086,10 @@ extern "C" int od_create(const od_config* cfg, od_ctx** out) {
       (rc = dalloc(&c->slot_of, np * 4)) || (rc = dalloc(&c->list_ion, np * 4)) || (rc = dalloc(&c->err, 4)) ||
       (rc = dalloc(&c->rec, (size_t)c->rec_cap * std::max(1, cfg->n_dust) * sizeof(od_dust_record))) ||
       (rc = dalloc(&c->rowD, 3 * np * 8)) || (rc = setup_sym(c, cfg)))
+    return fail(rc);
+  // chunk partials of the row kernels (launch_pair), where they run
+  if (!c->tile && !c->sym && !(cfg->cutoff > 0.0) && c->n_chunks > 1 &&
+      (rc = dalloc(&c->Fpart, (size_t)c->n_chunks * 3 * np * 8)))
     return fail(rc);
   DevParams hp;
   fill_params(cfg, c->n_pad, &hp);
