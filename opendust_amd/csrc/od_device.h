@@ -131,64 +131,65 @@ __device__ __forceinline__ void pair32(float xi, float yi, float zi, float xj, f
 // The device library's exp, sqrt and division also serve denormals, all signs
 // and exact rounding, and cost about 300 cycles per ordered pair and SIMD; the
 // law needs r2 in [1e-300, 1e31] and exp of a non-positive number.
-//   rsqrt, 1/x: the hardware's seeds (about 2^-24) and one third-order step
-//     each, y (1 + e/2 + 3 e^2/8) and z (1 + e + e^2); the error after the
-//     step is of order 2^-66, so rounding decides (about 1 ulp).
-//   exp(-d): -d = n ln2 + f (ln2 in two parts), e^f = 1 + f q(f) with q of
-//     degree 10 interpolating (e^f - 1)/f at the Chebyshev nodes of
-//     |f| <= ln2/2 (relative error 1e-17), scaled by 2^n; n saturates in the
-//     conversion, so a parked ion (d ~ 1e15) gives exactly 0.
+//   sqrt, 1/x: the hardware's rsqrt and reciprocal seeds (about 2^-24) and one
+//     third-order step each, r (1 + e/2 + 3 e^2/8) and z (1 + e + e^2); the
+//     error after the step is of order 2^-66, so rounding decides (about 1 ulp).
+//   2^-r: -r = n + f exactly, 2^f = 1 + f q(f) with q of degree 10 interpolating
+//     (2^f - 1)/f at the Chebyshev nodes of |f| <= 1/2 (relative error 2e-17),
+//     scaled by 2^n; n saturates in the conversion, so a parked ion (r ~ 1e15)
+//     gives exactly 0.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double rsqrt64(double r2) {
-  const double y = __builtin_amdgcn_rsq(r2);
-  const double e = fma(-(r2 * y), y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
 __device__ __forceinline__ double recip64(double b) {
   const double z = __builtin_amdgcn_rcp(b);
   const double e = fma(-b, z, 1.0);
   return fma(z, fma(e, e, e), z);
 }
 
-__device__ __forceinline__ double exp_neg64(double d) {
-  const double n = __builtin_rint(d * -1.4426950408889634);
-  double f = fma(n, -0.6931471805599453, -d);
-  f = fma(n, -2.3190468138462996e-17, f);
-  double q = 0x1.af4ddd84882fep-26;
-  q = fma(q, f, 0x1.28a2c0a7209fbp-22);
-  q = fma(q, f, 0x1.71de02375656cp-19);
-  q = fma(q, f, 0x1.a019a66a75dd4p-16);
-  q = fma(q, f, 0x1.a01a01abe62ddp-13);
-  q = fma(q, f, 0x1.6c16c17f43a58p-10);
-  q = fma(q, f, 0x1.11111111100dfp-7);
-  q = fma(q, f, 0x1.55555555520afp-5);
-  q = fma(q, f, 0x1.5555555555557p-3);
-  q = fma(q, f, 0x1.0000000000005p-1);
-  q = fma(q, f, 1.0);
+__device__ __forceinline__ double exp2_neg64(double r) {
+  const double n = __builtin_rint(-r);
+  const double f = -r - n;
+  double q = 0x1.e9d3fe3952179p-32;
+  q = fma(q, f, 0x1.e6063f7217bc6p-28);
+  q = fma(q, f, 0x1.b524fae627834p-24);
+  q = fma(q, f, 0x1.62bfd47773353p-20);
+  q = fma(q, f, 0x1.ffcbfc670dcd4p-17);
+  q = fma(q, f, 0x1.430913096fd9fp-13);
+  q = fma(q, f, 0x1.5d87fe78a5276p-10);
+  q = fma(q, f, 0x1.3b2ab6fba1ddap-7);
+  q = fma(q, f, 0x1.c6b08d704a0c2p-5);
+  q = fma(q, f, 0x1.ebfbdff82c598p-3);
+  q = fma(q, f, 0x1.62e42fefa39efp-1);
   q = fma(q, f, 1.0);
   int i;
   asm("v_cvt_i32_f64 %0, %1" : "=v"(i) : "v"(n));
   return __builtin_amdgcn_ldexp(q, i);
 }
 
-// FP64 form in lambda units: h = exp(-r) (1/r) z (1 + z), z = 1/(r + rho0)
-// (-U'/r of U = exp(-r)/(r + rho0)); F_i = -(kqq/lambda^2) sum_j h d.
-__device__ __forceinline__ double pair64_h(double r2, double rho0) {
-  const double y = rsqrt64(r2);
-  const double r = r2 * y;
-  const double z = recip64(r + rho0);
-  const double yz = y * z;
-  return exp_neg64(r) * fma(yz, z, yz);
+// sqrt(r2), r2 >= 1e-300: the rsqrt seed's third-order step on r = r2 y
+__device__ __forceinline__ double sqrt64(double r2) {
+  const double y = __builtin_amdgcn_rsq(r2);
+  const double t = r2 * y;
+  const double e = fma(-t, y, 1.0);
+  return fma(t, e * fma(e, 0.375, 0.5), t);
+}
+
+constexpr double LN2_64 = 0.6931471805599453;  // 1 / log2 e
+
+// FP64 form, in the FP32 form's units (r_D_e / log2 e; a = rho0 L): w =
+// 1/(r (r + a)), h = 2^-r w (r w + 1/L); F_i = -(kqq/lambda^2) L^2 sum_j h d.
+__device__ __forceinline__ double pair64_h(double r2, double a) {
+  const double r = sqrt64(r2);
+  const double w = recip64(fma(a, r, r2));
+  return exp2_neg64(r) * (w * fma(r, w, LN2_64));
 }
 
 __device__ __forceinline__ void pair64(double xi, double yi, double zi, double xj, double yj, double zj,
-                                       double rho0, double& ax, double& ay, double& az) {
+                                       double a, double& ax, double& ay, double& az) {
   const double dx = xj - xi;
   const double dy = yj - yi;
   const double dz = zj - zi;
   const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, EPS64)));
-  const double h = pair64_h(r2, rho0);
+  const double h = pair64_h(r2, a);
   ax = fma(h, dx, ax);
   ay = fma(h, dy, ay);
   az = fma(h, dz, az);
@@ -228,42 +229,26 @@ __device__ __forceinline__ void pair32_cut(float xi, float yi, float zi, float x
 
 // the FP64 law's h inside the cutoff (SW: switched)
 template <bool SW>
-__device__ __forceinline__ double pair64_cut_h(double r2, double rho0, double rs, double invw) {
-  const double y = rsqrt64(r2);
-  const double r = r2 * y;
-  const double e = exp_neg64(r);
-  const double z = recip64(r + rho0);
-  const double yz = y * z;
-  double h = e * fma(yz, z, yz);
-  if constexpr (SW) {
-    const double x = fmin(fmax((r - rs) * invw, 0.0), 1.0);
-    const double x2 = x * x, omx = 1.0 - x;
-    const double S = fma(x2 * x, fma(x, fma(x, -6.0, 15.0), -10.0), 1.0);
-    h = fma(h, S, e * yz * (30.0 * x2 * omx * omx * invw));
-  }
-  return h;
+__device__ __forceinline__ double pair64_cut_h(double r2, double a, double rs, double invw) {
+  if constexpr (!SW) return pair64_h(r2, a);
+  const double r = sqrt64(r2);
+  const double w = recip64(fma(a, r, r2));
+  const double ew = exp2_neg64(r) * w;
+  const double x = fmin(fmax((r - rs) * invw, 0.0), 1.0);
+  const double x2 = x * x, omx = 1.0 - x;
+  const double S = fma(x2 * x, fma(x, fma(x, -6.0, 15.0), -10.0), 1.0);
+  return fma(ew * fma(r, w, LN2_64), S, ew * (30.0 * x2 * omx * omx * invw));
 }
 
 __device__ __forceinline__ void pair64_cut(double xi, double yi, double zi, double xj, double yj, double zj,
-                                           double rho0, bool sw, double rc, double rs, double invw, double& ax,
+                                           double a, bool sw, double rc2, double rs, double invw, double& ax,
                                            double& ay, double& az) {
   const double dx = xj - xi;
   const double dy = yj - yi;
   const double dz = zj - zi;
   const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, EPS64)));
-  const double y = rsqrt64(r2);
-  const double r = r2 * y;
-  if (!(r < rc)) return;
-  const double e = exp_neg64(r);
-  const double z = recip64(r + rho0);
-  const double yz = y * z;
-  double h = e * fma(yz, z, yz);
-  if (sw) {
-    const double x = fmin(fmax((r - rs) * invw, 0.0), 1.0);
-    const double x2 = x * x, omx = 1.0 - x;
-    const double S = fma(x2 * x, fma(x, fma(x, -6.0, 15.0), -10.0), 1.0);
-    h = fma(h, S, e * yz * (30.0 * x2 * omx * omx * invw));
-  }
+  if (!(r2 < rc2)) return;
+  const double h = sw ? pair64_cut_h<true>(r2, a, rs, invw) : pair64_h(r2, a);
   ax = fma(h, dx, ax);
   ay = fma(h, dy, ay);
   az = fma(h, dz, az);

@@ -89,14 +89,14 @@ struct DevParams {
   uint32_t dust_mask;  // flag bits of the dusts
   uint64_t seed;
   double R, H, half_H, dt, half_dt, m_s, v_T, v_fl, lam;
-  double pos_scale;   // nm -> kernel units (FP32: L/lambda, FP64: 1/lambda)
+  double pos_scale;   // nm -> kernel units (L/lambda, L = log2 e)
   double pair_scale;  // kernel accumulator -> kJ/mol/nm
   float a32, linv32;
-  double rho0;
-  // truncation (cutoff mode): FP32 values in L/lambda units, FP64 in lambda units
+  double a64;
+  // truncation (cutoff mode), in the kernels' units
   int use_cut, use_switch;
   float rc32, rs32, invw32, rc2_32;
-  double rc64, rs64, invw64;
+  double rc64, rs64, invw64, rc2_64;
   // cell grid (nm): columns of col_w in x and y, slabs of slab_h in z
   double col_w, slab_h;
   int nx, ny, nz, n_cells;
@@ -166,9 +166,9 @@ template <>
 __device__ __forceinline__ void pair_acc<double>(const DevParams& P, const double4& i, const double4& j,
                                                  Acc<double>& ax, Acc<double>& ay, Acc<double>& az) {
   if (!P.use_cut)
-    pair64(i.x, i.y, i.z, j.x, j.y, j.z, P.rho0, ax.a, ay.a, az.a);
+    pair64(i.x, i.y, i.z, j.x, j.y, j.z, P.a64, ax.a, ay.a, az.a);
   else
-    pair64_cut(i.x, i.y, i.z, j.x, j.y, j.z, P.rho0, P.use_switch != 0, P.rc64, P.rs64, P.invw64, ax.a, ay.a,
+    pair64_cut(i.x, i.y, i.z, j.x, j.y, j.z, P.a64, P.use_switch != 0, P.rc2_64, P.rs64, P.invw64, ax.a, ay.a,
                az.a);
 }
 
@@ -187,11 +187,11 @@ struct PlainLaw<float> {
 };
 template <>
 struct PlainLaw<double> {
-  double rho0;
-  __device__ explicit PlainLaw(const DevParams& P) : rho0(P.rho0) {}
+  double a;
+  __device__ explicit PlainLaw(const DevParams& P) : a(P.a64) {}
   __device__ __forceinline__ void operator()(const double4& i, const double4& j, Acc<double>& ax, Acc<double>& ay,
                                              Acc<double>& az) const {
-    pair64(i.x, i.y, i.z, j.x, j.y, j.z, rho0, ax.a, ay.a, az.a);
+    pair64(i.x, i.y, i.z, j.x, j.y, j.z, a, ax.a, ay.a, az.a);
   }
 };
 
@@ -402,22 +402,18 @@ static int fill_params(const od_config* c, int n_pad, DevParams* P, CellGrid gri
   P->v_T = c->v_T;
   P->v_fl = c->v_fl;
   P->lam = c->r_D_e;
-  P->rho0 = c->r_0 / c->r_D_e;
+  P->a64 = c->r_0 / c->r_D_e * L;
   const double C = c->kqq / (c->r_D_e * c->r_D_e);  // kJ/mol/nm
-  if (c->precision == OD_PREC_FP32C) {
-    P->pos_scale = L / c->r_D_e;
-    P->pair_scale = -C * L * L;
-  } else {
-    P->pos_scale = 1.0 / c->r_D_e;
-    P->pair_scale = -C;
-  }
+  P->pos_scale = L / c->r_D_e;
+  P->pair_scale = -C * L * L;
   if (c->cutoff > 0.0) {
     P->use_cut = 1;
     P->use_switch = (c->switch_dist > 0.0 && c->switch_dist < c->cutoff) ? 1 : 0;
     const double rc = c->cutoff / c->r_D_e, rs = P->use_switch ? c->switch_dist / c->r_D_e : rc;
-    P->rc64 = rc;
-    P->rs64 = rs;
-    P->invw64 = P->use_switch ? 1.0 / (rc - rs) : 0.0;
+    P->rc64 = rc * L;
+    P->rc2_64 = rc * L * (rc * L);
+    P->rs64 = rs * L;
+    P->invw64 = P->use_switch ? 1.0 / ((rc - rs) * L) : 0.0;
     P->rc32 = (float)(rc * L);
     P->rc2_32 = (float)(rc * L * rc * L);
     P->rs32 = (float)(rs * L);
@@ -439,7 +435,7 @@ static int fill_params(const od_config* c, int n_pad, DevParams* P, CellGrid gri
     P->ny = P->nx;
     P->n_fwd = cell_offsets(grid, P->off);
   }
-  P->a32 = (float)(P->rho0 * L);
+  P->a32 = (float)P->a64;
   P->linv32 = (float)(1.0 / L);
   P->thr_top = c->thr_top;
   P->thr_side = c->use_bottom ? c->thr_side : 4294967296ull;
@@ -1194,7 +1190,7 @@ static int launch_pair(od_ctx* c, const void* pi, const void* pj, double* F, boo
                        c->n_pad, c->n_chunks, c->chunk_len, a, linv, -C * L * L, out);
   } else {
     hipLaunchKernelGGL(k_pair64<1>, dim3(grid), dim3(256), 0, c->stream, (const double4*)pi, (const double4*)pj,
-                       c->n_pad, c->n_chunks, c->chunk_len, c->cfg.r_0 / c->cfg.r_D_e, -C, out);
+                       c->n_pad, c->n_chunks, c->chunk_len, c->cfg.r_0 / c->cfg.r_D_e * L, -C * L * L, out);
   }
   if (timed) HIPCHK(hipEventRecord(c->ev1, c->stream));
   if (c->n_chunks > 1) {
@@ -1409,7 +1405,7 @@ static int launch_step(od_ctx* c, bool timed) {
 template <class T>
 static int load_positions_t(od_ctx* c, const double* X, void* pi, void* pj) {
   using PV = typename Pos<T>::V;
-  const double s = (c->prec == OD_PREC_FP32C) ? 1.4426950408889634 / c->cfg.r_D_e : 1.0 / c->cfg.r_D_e;
+  const double s = 1.4426950408889634 / c->cfg.r_D_e;
   hipLaunchKernelGGL(k_load_pos<T>, dim3(c->nb), dim3(256), 0, c->stream, X, c->n, c->n_pad, s, (PV*)pi, (PV*)pj);
   return OD_OK;
 }
