@@ -532,7 +532,7 @@ static int tile_build(TilePlan* t, const TileSims& sims, bool fp32) {
   groups.push_back({0, 0, u, 0});
   t->n_units = u;
   t->n_sub = (int)subs.size();
-  t->per = std::max(1, (u + TILE_WGS - 1) / TILE_WGS);
+  t->per = tile_per(u, t->nw, fp32);
   t->n_wg = (u + t->per - 1) / t->per;
   std::vector<int> wg(t->n_wg);
   for (int b = 0, g = 0; b < t->n_wg; ++b) {
