@@ -234,10 +234,14 @@ __device__ __forceinline__ double pair64_cut_h(double r2, double a, double rs, d
   const double r = sqrt64(r2);
   const double w = recip64(fma(a, r, r2));
   const double ew = exp2_neg64(r) * w;
-  const double x = fmin(fmax((r - rs) * invw, 0.0), 1.0);
-  const double x2 = x * x, omx = 1.0 - x;
-  const double S = fma(x2 * x, fma(x, fma(x, -6.0, 15.0), -10.0), 1.0);
-  return fma(ew * fma(r, w, LN2_64), S, ew * (30.0 * x2 * omx * omx * invw));
+  double h = ew * fma(r, w, LN2_64);
+  if (r > rs) {
+    const double x = (r - rs) * invw;
+    const double x2 = x * x, omx = 1.0 - x;
+    const double S = fma(x2 * x, fma(x, fma(x, -6.0, 15.0), -10.0), 1.0);
+    h = fma(h, S, ew * (30.0 * x2 * omx * omx * invw));
+  }
+  return h;
 }
 
 __device__ __forceinline__ void pair64_cut(double xi, double yi, double zi, double xj, double yj, double zj,

@@ -324,14 +324,17 @@ __device__ __forceinline__ void sym_tile_lds(SymT<MT>& T, const float4* ls, floa
         const float w = __builtin_amdgcn_rcpf(__builtin_fmaf(L.a, r, r2));
         const float t = __builtin_fmaf(r, w, L.linv);
         float h = e * w * t;
-        if constexpr (CUT == 2) {
-          const float x = __builtin_fminf(__builtin_fmaxf((r - L.rs) * L.invw, 0.0f), 1.0f);
-          const float x2 = x * x;
-          const float Sx = __builtin_fmaf(x2 * x, __builtin_fmaf(x, __builtin_fmaf(x, -6.0f, 15.0f), -10.0f), 1.0f);
-          const float omx = 1.0f - x;
-          const float dS = -30.0f * x2 * omx * omx * L.invw;
-          h = __builtin_fmaf(h, Sx, -(e * w * dS));
-        }
+        // the switch acts beyond rs only: skipped where no lane's pair is there
+        if constexpr (CUT == 2)
+          if (r > L.rs) {
+            const float x = (r - L.rs) * L.invw;
+            const float x2 = x * x;
+            const float Sx =
+                __builtin_fmaf(x2 * x, __builtin_fmaf(x, __builtin_fmaf(x, -6.0f, 15.0f), -10.0f), 1.0f);
+            const float omx = 1.0f - x;
+            const float dS = -30.0f * x2 * omx * omx * L.invw;
+            h = __builtin_fmaf(h, Sx, -(e * w * dS));
+          }
         T.ax[k] = __builtin_fmaf(h, dx, T.ax[k]);
         T.ay[k] = __builtin_fmaf(h, dy, T.ay[k]);
         T.az[k] = __builtin_fmaf(h, dz, T.az[k]);
