@@ -918,7 +918,7 @@ static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
   if (c->list) {
     // one allocation for the tables, one for the partial sums
     const size_t ne = (size_t)c->n_entries + 1;
-    const size_t b_tp = ((size_t)CL_WAVES + c->max_items) * 3 * CL_G * 8;
+    const size_t b_tp = ((size_t)cl_waves(c->n) + c->max_items) * 3 * CL_G * 8;
     if ((rc = dalloc(&c->cl_rng, ne * 16 + 4)) || (rc = dalloc(&c->rc4_cell, np * 4)) ||
         (rc = dalloc(&c->cl_tp, b_tp + (size_t)c->cl_cap * 192 * (c->prec == OD_PREC_FP32C ? 4 : 8))))
       return rc;
@@ -1265,11 +1265,11 @@ static int launch_forces_t(od_ctx* c, const double* X, const void* pos, const ui
   const int* n_units = c->list ? c->cl_total : nullptr;
   if (c->list) {
     // the kernels after these two return at once unless the units overflow
-    hipLaunchKernelGGL((sw ? k_cell_list<T, 2> : k_cell_list<T, 1>), dim3(CL_WAVES), dim3(64), 0, c->stream, c->dP,
-                       (const PV*)c->spos, c->skey, c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries,
+    hipLaunchKernelGGL((sw ? k_cell_list<T, 2> : k_cell_list<T, 1>), dim3(cl_waves(c->n)), dim3(64), 0, c->stream,
+                       c->dP, (const PV*)c->spos, c->skey, c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries,
                        n_units, c->cl_cap, c->cl_tp, (T*)c->cl_sp);
     hipLaunchKernelGGL(k_cell_list_reduce<T>, dim3(c->n_pad / 256), dim3(256), 0, c->stream, c->dP, c->skey, c->sval,
-                       c->cell_start, c->item_off, c->cl_rng, c->cl_u0, n_units, c->cl_cap, CL_WAVES,
+                       c->cell_start, c->item_off, c->cl_rng, c->cl_u0, n_units, c->cl_cap, cl_waves(c->n),
                        (const double*)c->cl_tp, (const T*)c->cl_sp, F);
   }
   if constexpr (std::is_same<T, float>::value) {
