@@ -1316,7 +1316,7 @@ static int launch_step_t(od_ctx* c, bool timed) {
   hipLaunchKernelGGL(k_kick_drift<T>, dim3(nb), dim3(256), 0, c->stream, c->dP, (const int*)nullptr, c->X, c->V,
                      c->F, c->q, c->st, (PV*)c->pi, (PV*)c->pj, c->flags, c->block_cnt, c->err);
   mark(c, OD_STAGE_LIST);
-  const bool few = nb <= FEW_BLOCKS;
+  const bool few = few_blocks<T>(nb);
   if (few) {
     hipLaunchKernelGGL(k_scan_list<T>, dim3(nb), dim3(256), 0, c->stream, c->flags, c->block_cnt, c->block_off,
                        c->n_flag, c->n, (const PV*)c->pi, c->slot_of, c->list_ion, (PV*)c->list_old);
