@@ -6,13 +6,18 @@
 //
 //   k_kick_drift   collisions, first half-kick, drift, absorption/outflow flags
 //   k_scan/k_list  ordered compaction of the flagged ions (ion-index order)
-//   k_pair32/64    ion-ion force at the drifted positions; flagged ions are
+//   k_pair_tile, k_pair32_sym, k_cell_list, ...
+//                  ion-ion force at the drifted positions; flagged ions are
 //                  parked far away as sources, so this is the sum over kept ions
 //   k_kick2        + flagged-source correction, second half-kick, absorbed
 //                  counts and momenta, Philox reinjection, orbit sums
 //   k_rows         full force rows of the reinjected ions at their new place
 //   k_inflow       force of the reinjected ions on everybody else
 //   k_dust         FP64 reductions, charge update, per-step dust records
+//
+// Up to FEW_BLOCKS blocks of ions (4 times fewer in FP64) some of these share a
+// launch: k_scan_list; the absorbed ions' rows ride on k_tile_reduce; k_step_end
+// is k_rows, k_inflow and k_dust.
 //
 // The reference evaluates the ion-ion force twice per step (OpenMM recomputes
 // forces after the reinjection writes x).  Here the second evaluation costs
@@ -1521,6 +1526,10 @@ extern "C" int od_set_step(od_ctx* c, int64_t step) {
   return OD_OK;
 }
 
+// Steps per captured graph.  Capturing and instantiating costs a new context
+// about 2.5 us per kernel, a replay some microseconds.
+constexpr int GRAPH_STEPS = 16;
+
 static int build_graph(od_ctx* c, int steps) {
   if (c->gexec && c->graph_steps == steps) return OD_OK;
   if (c->gexec) {
@@ -1563,7 +1572,7 @@ extern "C" int od_run(od_ctx* c, int64_t nsteps, od_dust_record* out, int32_t fl
     HIPCHK(hipMemcpyAsync(c->st + 1, &base, 4, hipMemcpyHostToDevice, c->stream));
     int left = chunk;
     if (graph && chunk >= 4) {
-      const int gs = std::min(chunk, 32);
+      const int gs = std::min(chunk, GRAPH_STEPS);
       CHKRET(build_graph(c, gs));
       while (left >= gs) {
         HIPCHK(hipGraphLaunch(c->gexec, c->stream));
