@@ -46,10 +46,10 @@ extern "C" {
 #define OD_PREC_FP32C 0 /* FP32 pair arithmetic, compensated (Kahan) per-ion sums */
 #define OD_PREC_FP64 1  /* plain FP64 pair arithmetic */
 
-/* all-pairs kernel (FP32 path; the FP64 path always uses the row kernel) */
-#define OD_PAIR_AUTO 0 /* symmetric when the problem is large enough, else rows */
+/* all-pairs kernel */
+#define OD_PAIR_AUTO 0 /* every unordered pair once: wave tiles (FP64; FP32c below 2^18 ions), else blocks */
 #define OD_PAIR_ROWS 1 /* every ordered pair, one target row per thread */
-#define OD_PAIR_SYM 2  /* every unordered pair once (Newton's third law) */
+#define OD_PAIR_SYM 2  /* every unordered pair once (Newton's third law); FP32c: 1024-ion blocks (sym_*) */
 #define OD_PAIR_CELL 3 /* reported by od_pair_info when a cutoff is set: cell list + stencil */
 
 /* charge methods (opendust.py:1120, :1153; any other string keeps q) */
@@ -82,7 +82,8 @@ typedef struct od_config {
   int32_t precision;     /* OD_PREC_* */
   int32_t device;        /* HIP device ordinal */
   int32_t use_bottom;    /* reference applies the bottom-face selects only if p_b != 0 (opendust.py:939) */
-  int32_t j_split;       /* source chunks of the row pair kernel; 0 = automatic */
+  int32_t j_split;       /* source chunks of the row pair kernel (> 0 selects it where it is the
+                            automatic kernel of FP64 or of small FP32c contexts); 0 = automatic */
   int32_t pair_mode;     /* OD_PAIR_*: which all-pairs kernel */
   int32_t sym_chunk;     /* symmetric kernel: 1024-ion source blocks per workgroup; 0 = automatic */
   int32_t sim_id;        /* Philox counter word 2 (index of the simulation in a sweep; 0 alone) */
@@ -93,7 +94,8 @@ typedef struct od_config {
                             11 with at least 2048 work-groups, else 3).  Cutoff mode, FP32c: the
                             symmetric cell kernel's 64-target sub-blocks per wave, 1, 2, 3 = 1, 2, 4
                             with sources rotated through registers, 4, 5, 6 = 1, 2, 4 with sources
-                            read from LDS; 0 = 5 */
+                            read from LDS; 0 = the evenly split cell list, on a grid that follows the
+                            ion density */
   int32_t sym_band_mib;  /* symmetric kernel: partials per band of rows of its triangular schedule, MiB;
                             0 = 48 GB (larger schedules, about 2^21 ions and up, run in several bands) */
   uint64_t seed;         /* Philox4x32-10 key */
@@ -230,8 +232,8 @@ int od_stage_timing(od_ctx* ctx, double* ms, int64_t* steps, int32_t reset);
 
 /* Which all-pairs kernel the context runs (OD_PAIR_ROWS or OD_PAIR_SYM) and
  * how many ordered ion pairs its main launch (the one OD_RUN_PROFILE_PAIR
- * times) covers: N(N-1) for rows, N(N-1) minus the intra-block pairs for the
- * symmetric kernel.  No counterpart in the reference (measurement support). */
+ * times) covers: N(N-1) for rows and for wave tiles, N(N-1) minus the
+ * intra-block pairs for the symmetric block kernel.  No counterpart in the reference (measurement support). */
 int od_pair_info(od_ctx* ctx, int32_t* mode, int64_t* pairs_per_launch);
 
 /* The symmetric kernel's current schedule: source blocks per work-group,
@@ -239,13 +241,16 @@ int od_pair_info(od_ctx* ctx, int32_t* mode, int64_t* pairs_per_launch);
  * of bands of rows its triangular schedule runs in (od_config.sym_band_mib);
  * 0, 0 and 0 when the context does not run it.  Cutoff mode, FP32c: 0, the
  * symmetric cell kernel's variant (1, 2, 3: 1, 2, 4 target sub-blocks per
- * wave) and 0.  Measurement support. */
+ * wave; 0: the evenly split cell list) and 0.  Measurement support. */
 int od_sym_choice(od_ctx* ctx, int32_t* sym_chunk, int32_t* sym_tile, int32_t* bands);
 
 /* Autotuner of the symmetric FP32 pair kernel (contexts that run it; others
- * return *sym_chunk = *sym_tile = 0 and change nothing; cutoff mode, FP32c:
- * it times the symmetric cell kernel's six variants on the current ions, keeps
- * the fastest and returns *sym_chunk = 0, *sym_tile = the variant).  It times the whole
+ * return *sym_chunk = *sym_tile = 0 and change nothing; an FP32c context of
+ * wave tiles with at least 2^15 ions compares them with the best schedule found
+ * and keeps the faster, 0 and 0 for the tiles; cutoff mode, FP32c, with a
+ * variant fixed by sym_tile: it times the symmetric cell kernel's six variants
+ * on the current ions, keeps the fastest and returns *sym_chunk = 0, *sym_tile
+ * = the variant).  It times the whole
  * pair evaluation `reps` times per candidate on the current ions: first 1, 2,
  * 4, 8, 16 and 32 source blocks per work-group with the configured kernel
  * variant, then every kernel variant (tile shape: 4, 8 or 16 64-target
@@ -284,9 +289,9 @@ int od_get_cells(od_ctx* ctx, int32_t* cell_of_ion, int32_t* sorted_ions, int64_
 /* Cutoff mode only, for the current cell list (measurement support):
  * ordered ion pairs within the cutoff, and the ordered pair terms the cell
  * kernel evaluates, padding included (FP64: 64 lanes x the sources of the
- * slab ranges of each 64-target chunk; FP32c symmetric kernel: two terms per
- * evaluated pair slot, force and reaction, one per slot of a group's own
- * pairs). */
+ * slab ranges of each 64-target chunk; FP32c, and FP64 on the evenly split
+ * list: two terms per pair slot, force and reaction, one per slot of a
+ * group's own pairs; slots whose distance test skips them count too). */
 int od_cutoff_pair_count(od_ctx* ctx, int64_t* in_range, int64_t* candidates);
 
 /* Diagnostics of the last step (for parity tests): per-ion flag word
@@ -380,7 +385,9 @@ int od_batch_pair_timing(od_batch* b, double* total_ms, int64_t* launches, int64
                          int32_t reset);
 
 /* od_tune for a batch (all simulations share one schedule; the choice is
- * fixed through the first configuration's sym_chunk and sym_tile).  Call
+ * fixed through the first configuration's sym_chunk and sym_tile).  A batch of
+ * wave tiles (the automatic choice below 2^18 ions per simulation) runs the
+ * schedule found instead.  Call
  * after the od_batch_set_ions calls; the next od_batch_run recomputes the
  * forces. */
 int od_batch_tune(od_batch* b, int32_t reps, int32_t* sym_chunk, int32_t* sym_tile);
