@@ -224,8 +224,10 @@ def cutoff_leg(steps):
         "cell_kernel_tflops_alg": in_range * FLOP_PER_PAIR / (ms / max(nl, 1) * 1e-3) / 1e12,
         "cell_kernel_frac_of_fp32_peak": in_range * FLOP_PER_PAIR / (ms / max(nl, 1) * 1e-3) / 1e12
                                          / FP32_PEAK_TFLOPS,
-        "cell_kernel_variant": {"sym_tile": variant, "targets_per_lane": {1: 1, 2: 2, 3: 4, 4: 1, 5: 2, 6: 4}.get(variant),
-                                "sources_from_lds": variant in (4, 5, 6)},
+        # variant 0: the evenly split cell list (its own grid; "grid" is od_get_cells')
+        "cell_kernel_variant": {"sym_tile": variant,
+                                "targets_per_lane": {0: 2, 1: 1, 2: 2, 3: 4, 4: 1, 5: 2, 6: 4}.get(variant),
+                                "sources_from_lds": variant in (0, 4, 5, 6)},
         "grid": {"dims": list(dims), "cells": n_cells, "radix_passes": passes},
         "stage_ms": st,
         "hbm_stages": hbm_stages(st, 2 ** 22, dict(STAGE_BYTES_PER_ION_CUTOFF, cells=cb)),
@@ -486,13 +488,16 @@ def main():
                             if (mode == engine.PAIR_SYM and N == 2 ** 20 and tile) else (None, None))
     log("fp32c: %.2f ms/step, pair kernel %.2f ms, %.3e pairs/s" % (ms_per_step, kernel_ms, value))
 
-    # FP64 GPU path and FP32c-vs-FP64 dust force error from the same state
+    # plain FP64 GPU path (every ordered pair, the row kernel), the automatic FP64 kernel, and the
+    # FP32c-vs-FP64 dust force error from the same state
     fp64 = None
     if args.fp64_steps > 0:
         step_idx = args.warmup + args.steps
         cfg64 = od.make_config(od.reinjection_tables(), od.alphaTrap, precision="fp64", seed=od.seed)
+        rows64 = engine.Config.from_buffer_copy(cfg64)
+        rows64.pair_mode = engine.PAIR_ROWS
         res = {}
-        for prec, c in (("fp64", cfg64), ("fp32c", cfg)):
+        for prec, c in (("fp64", rows64), ("fp64_auto", cfg64), ("fp32c", cfg)):
             e = engine.Engine(c)
             e.set_ions(x_mid, v_mid)
             e.set_dust_charges(q_mid)
@@ -510,6 +515,8 @@ def main():
             "ms_per_step": t64 / args.fp64_steps * 1e3,
             "pair_interactions_per_s": pairs_step * args.fp64_steps / t64,
             "fp32c_speedup": value / (pairs_step * args.fp64_steps / t64),
+            "auto_ms_per_step": res["fp64_auto"][0] / args.fp64_steps * 1e3,
+            "auto_pair_interactions_per_s": pairs_step * args.fp64_steps / res["fp64_auto"][0],
             "dust_force_rel_err_first_step": float(np.linalg.norm(fo32 - fo64) / np.linalg.norm(fo64)),
         }
         log("fp64:", fp64)
@@ -565,7 +572,7 @@ def main():
             "traffic": traffic,
             "traffic_source": traffic_src,
             "traffic_unit": "bytes per launch",
-            "kernel": "k_pair32_sym" if mode == engine.PAIR_SYM else "k_pair32<2>",
+            "kernel": ("k_pair32_sym" if tile else "k_pair_tile") if mode == engine.PAIR_SYM else "k_pair32<2>",
             "kernel_ms": kernel_ms,
             "flop_per_pair": FLOP_PER_PAIR,
             "pairs_per_launch": pairs_launch,
