@@ -811,7 +811,8 @@ static double cell_list_units(const od_config* cfg, int n, CellGrid g) {
 // share inside the cylinder (4 x 4 points each; beyond 64 columns across, all
 // as full).  Force evaluation, columns cutoff/4 and slabs cutoff/16 -> this:
 // 130001 ions FP64 1.30 -> 0.47 ms (pair terms per in-range pair 15.9 ->
-// 5.4), FP32c 32768 ions 0.24 -> 0.06, 262144 1.07 -> 0.55, 2^20 5.6 -> 5.0;
+// 5.4), FP32c 32768 ions 0.24 -> 0.06, 262144 1.07 -> 0.55, 2^20 5.6 -> 5.0
+// (with the pairs out of range skipped and cl_waves 0.39, 0.05, 0.46 and 3.8);
 // at 2^22 the choice is columns of cutoff/4.
 constexpr double CELL_ENTRY_COST = 24.0;
 static CellGrid choose_grid(const od_config* cfg, int n) {
