@@ -1274,8 +1274,8 @@ static int launch_forces_t(od_ctx* c, const double* X, const void* pos, const ui
     hipLaunchKernelGGL((sw ? k_cell_list<T, 2> : k_cell_list<T, 1>), dim3(cl_waves(c->n)), dim3(64), 0, c->stream,
                        c->dP, (const PV*)c->spos, c->skey, c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries,
                        n_units, c->cl_cap, c->cl_tp, (T*)c->cl_sp);
-    hipLaunchKernelGGL(k_cell_list_reduce<T>, dim3(c->n_pad / 256), dim3(256), 0, c->stream, c->dP, c->skey, c->sval,
-                       c->cell_start, c->item_off, c->cl_rng, c->cl_u0, n_units, c->cl_cap, cl_waves(c->n),
+    hipLaunchKernelGGL(k_cell_list_reduce<T>, dim3(c->n_pad / 64), dim3(64 * REDUCE_PARTS), 0, c->stream, c->dP,
+                       c->skey, c->sval, c->cell_start, c->item_off, c->cl_rng, c->cl_u0, n_units, c->cl_cap, cl_waves(c->n),
                        (const double*)c->cl_tp, (const T*)c->cl_sp, F);
   }
   if constexpr (std::is_same<T, float>::value) {
