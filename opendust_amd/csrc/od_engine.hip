@@ -38,6 +38,7 @@
 #include <vector>
 
 #include "od_device.h"
+#include "od_scan.h"
 #include "od_sym_tile.h"
 
 using namespace od;
@@ -869,10 +870,13 @@ static CellGrid choose_grid(const od_config* cfg, int n) {
 // spread's units, fit CELL_LIST_MAX_BYTES, unless the configuration fixes a
 // variant of k_pair32_symcol.
 constexpr double CELL_LIST_MAX_BYTES = 24e9;
+// below COUNT_MAX, so a unit count that saturated is over every capacity
+constexpr int CELL_LIST_MAX_UNITS = 1000000000;
+static_assert(CELL_LIST_MAX_UNITS < COUNT_MAX, "a saturated unit count must exceed the capacity");
 static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, CellGrid g, int* cap) {
   const double units = 2.0 * cell_list_units(cfg, c->n, g) + 4096.0;
   const bool fp32 = c->prec == OD_PREC_FP32C;
-  *cap = (int)std::min(units, 1e9);
+  *cap = (int)std::min(units, (double)CELL_LIST_MAX_UNITS);
   if (fp32 && cfg->sym_tile > 0) return false;
   return units * 192.0 * (fp32 ? 4.0 : 8.0) <= CELL_LIST_MAX_BYTES;
 }
@@ -1207,7 +1211,7 @@ static int launch_pair(od_ctx* c, const void* pi, const void* pj, double* F, boo
   return OD_OK;
 }
 
-// exclusive scan of n ints (in -> out, sum -> total) on the context's stream
+// exclusive scan of n counts (in -> out, sum -> total, saturating) on the context's stream
 static void launch_scan(od_ctx* c, const int* in, int n, int* out, int* total) {
   if (n <= 16384) {
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->stream, in, n, out, total);
