@@ -512,6 +512,7 @@ static void free_ctx(od_ctx* c) {
 template <class P>
 static int dalloc(P** p, size_t bytes) {
   hipError_t e = hipMalloc((void**)p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch check
   if (e != hipSuccess) return set_err(OD_ERR_HIP, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   return OD_OK;
 }
@@ -2154,17 +2155,26 @@ extern "C" int od_batch_tune(od_batch* b, int32_t reps, int32_t* sym_chunk, int3
     if (b->stale)
       hipLaunchKernelGGL(k_batch_load_pos<float>, dim3(b->nb), dim3(256), 0, b->stream, b->dP, b->blk_sim, b->X,
                          (float4*)b->pi, (float4*)b->pj);
-    if (b->tile) {
-      // the schedules tuned here are k_pair32_sym's: it replaces the wave tiles
-      if (b->blk_end_host.empty()) CHKRET(batch_setup_sym(b));
-      b->tile = 0;
-    }
+    // the schedules tuned here are k_pair32_sym's: it replaces the wave tiles,
+    // which stay if anything fails
+    const bool tiles = b->tile;
+    int rc = tiles ? batch_setup_sym(b) : OD_OK;
     double* Fs = nullptr;
-    CHKRET(dalloc(&Fs, (size_t)3 * b->n_tot * 8));
-    const int rc = tune_sym(b, b->blk_end_host, reps, [&]() { batch_pair<float>(b, false, Fs); }, &chosen, &var,
-                            1e300, SYM_BAND_BYTES);
-    (void)hipFree(Fs);
-    if (rc != OD_OK) return rc;
+    if (rc == OD_OK) rc = dalloc(&Fs, (size_t)3 * b->n_tot * 8);
+    if (rc == OD_OK) {
+      b->tile = 0;
+      rc = tune_sym(b, b->blk_end_host, reps, [&]() { batch_pair<float>(b, false, Fs); }, &chosen, &var, 1e300,
+                    SYM_BAND_BYTES);
+    }
+    if (rc != OD_OK) (void)hipStreamSynchronize(b->stream);
+    if (Fs) (void)hipFree(Fs);
+    if (rc != OD_OK) {
+      if (tiles) {
+        batch_release_sym(b);
+        b->tile = 1;
+      }
+      return rc;
+    }
     b->stale = true;  // the next run recomputes the forces with the chosen schedule
   }
   if (sym_chunk) *sym_chunk = chosen;

@@ -1,3 +1,5 @@
+import contextlib
+import ctypes
 import os
 import sys
 
@@ -24,6 +26,33 @@ def oracle_lib():
 def say(*a):
     """Progress line that names the case before a GPU step (flushed)."""
     print(*a, flush=True)
+
+
+@contextlib.contextmanager
+def gpu_memory_left(left):
+    """Holds all device memory but `left` bytes (allocated, never touched)."""
+    from opendust_amd import engine
+
+    engine.load_library()
+    with open("/proc/self/maps") as f:
+        path = next(w.split()[-1] for w in f if "libamdhip64" in w)
+    hip = ctypes.CDLL(path)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    held = []
+    try:
+        while True:
+            assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            take = min(free.value - left, 32 << 30)
+            if take < 1 << 20:
+                break
+            p = ctypes.c_void_p()
+            assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(take)) == 0
+            held.append(p)
+        say("  device memory left, GB:", round(free.value / 1e9, 2))
+        yield
+    finally:
+        for p in held:
+            hip.hipFree(p)
 
 
 def rel_err(a, b, floor=0.0):

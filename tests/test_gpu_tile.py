@@ -7,7 +7,7 @@ import io
 import numpy as np
 import pytest
 
-from conftest import say
+from conftest import gpu_memory_left, say
 
 pytestmark = pytest.mark.gpu
 
@@ -111,6 +111,40 @@ def test_tune_keeps_or_replaces_wave_tiles():
         assert np.linalg.norm(f1 - f0) <= 4e-6 * np.linalg.norm(f0)
     e.run(4, engine.RUN_GRAPH)
     e.close()
+
+
+def test_batch_tune_out_of_memory_keeps_wave_tiles():
+    """od_batch_tune on a GPU whose free memory does not hold the schedules it
+    would time (six simulations of 2^18 ions, 3.7 GB): an error, also when
+    called again, and the batch steps on with its wave tiles as if untuned."""
+    from opendust_amd import engine
+
+    cfg, x0, v0 = _setup(262080, "fp32c")
+    cfgs = []
+    for s in range(6):
+        cfgs.append(engine.Config.from_buffer_copy(cfg))
+        cfgs[s].sim_id = s
+
+    def batch():
+        b = engine.Batch(cfgs)
+        for s in range(6):
+            b.set_ions(s, x0, v0)
+        return b
+
+    b = batch()
+    with gpu_memory_left(2500 << 20):
+        for again in range(2):
+            say("batch tune out of memory, call", again)
+            with pytest.raises(RuntimeError, match="hipMalloc"):
+                b.tune(1)
+    rec = b.run(1)
+    x, v = b.get_ions(5)
+    b.close()
+    b = batch()
+    assert np.array_equal(b.run(1), rec)
+    x1, v1 = b.get_ions(5)
+    assert np.array_equal(x, x1) and np.array_equal(v, v1)
+    b.close()
 
 
 def test_fp64_pair_law_over_its_range():
