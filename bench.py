@@ -258,7 +258,7 @@ def sweep_leg(steps, seq_steps, n_sims=64, sweep_len=5000):
         b.set_ions(s_, x0, v0)
     chunk, tile = b.tune(3)
     log("sweep: autotuner chose %d source blocks per work-group, kernel variant %d %s"
-        % (chunk, tile, engine.sym_variants()[tile - 1]))
+        % (chunk, tile, engine.sym_variants()[tile - 1] if tile else "(wave tiles)"))
     b.run(3, engine.RUN_PROFILE_PAIR, records=False)
     b.pair_timing(reset=True)
     b.run(3, engine.RUN_PROFILE_PAIR, records=False)

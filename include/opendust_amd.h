@@ -386,10 +386,10 @@ int od_batch_pair_timing(od_batch* b, double* total_ms, int64_t* launches, int64
 
 /* od_tune for a batch (all simulations share one schedule; the choice is
  * fixed through the first configuration's sym_chunk and sym_tile).  A batch of
- * wave tiles (the automatic choice below 2^18 ions per simulation) runs the
- * schedule found instead.  Call
- * after the od_batch_set_ions calls; the next od_batch_run recomputes the
- * forces. */
+ * wave tiles (the automatic choice below 2^18 ions per simulation) compares
+ * them with the best schedule found and keeps the faster, 0 and 0 for the
+ * tiles, which also stay if the call fails.  Call after the od_batch_set_ions
+ * calls; the next od_batch_run recomputes the forces. */
 int od_batch_tune(od_batch* b, int32_t reps, int32_t* sym_chunk, int32_t* sym_tile);
 
 int od_batch_destroy(od_batch* b);

@@ -2155,26 +2155,30 @@ extern "C" int od_batch_tune(od_batch* b, int32_t reps, int32_t* sym_chunk, int3
     if (b->stale)
       hipLaunchKernelGGL(k_batch_load_pos<float>, dim3(b->nb), dim3(256), 0, b->stream, b->dP, b->blk_sim, b->X,
                          (float4*)b->pi, (float4*)b->pj);
-    // the schedules tuned here are k_pair32_sym's: it replaces the wave tiles,
-    // which stay if anything fails
+    // the schedules tuned here are k_pair32_sym's: wave tiles stay unless the
+    // best of them is faster, and if anything fails
     const bool tiles = b->tile;
-    int rc = tiles ? batch_setup_sym(b) : OD_OK;
-    double* Fs = nullptr;
-    if (rc == OD_OK) rc = dalloc(&Fs, (size_t)3 * b->n_tot * 8);
+    double *Fs = nullptr, tile_ms = 1e300, sym_ms = 1e300;
+    int rc = dalloc(&Fs, (size_t)3 * b->n_tot * 8);
+    auto evaluate = [&]() { batch_pair<float>(b, false, Fs); };
+    if (tiles && rc == OD_OK) {
+      evaluate();  // warm-up
+      rc = time_evaluations(b, reps, evaluate, &tile_ms);
+      if (rc == OD_OK) rc = batch_setup_sym(b);
+    }
     if (rc == OD_OK) {
       b->tile = 0;
-      rc = tune_sym(b, b->blk_end_host, reps, [&]() { batch_pair<float>(b, false, Fs); }, &chosen, &var, 1e300,
-                    SYM_BAND_BYTES);
+      rc = tune_sym(b, b->blk_end_host, reps, evaluate, &chosen, &var, 1e300, SYM_BAND_BYTES, &sym_ms);
     }
     if (rc != OD_OK) (void)hipStreamSynchronize(b->stream);
     if (Fs) (void)hipFree(Fs);
-    if (rc != OD_OK) {
-      if (tiles) {
-        batch_release_sym(b);
-        b->tile = 1;
-      }
-      return rc;
+    if (tiles && (rc != OD_OK || tile_ms <= sym_ms)) {
+      batch_release_sym(b);
+      b->tile = 1;
+      chosen = 0;
+      var = -1;
     }
+    if (rc != OD_OK) return rc;
     b->stale = true;  // the next run recomputes the forces with the chosen schedule
   }
   if (sym_chunk) *sym_chunk = chosen;

@@ -545,7 +545,8 @@ class Batch:
 
     def tune(self, reps=3):
         """Autotune the batch's symmetric kernel (see Engine.tune); returns
-        (sym_chunk, sym_tile), fixed through the first configuration."""
+        (sym_chunk, sym_tile), fixed through the first configuration; (0, 0)
+        if the batch keeps its wave tiles."""
         ch = ctypes.c_int32()
         tile = ctypes.c_int32()
         _check(self.lib.od_batch_tune(self._b, int(reps), ctypes.byref(ch), ctypes.byref(tile)), "od_batch_tune")

@@ -80,7 +80,7 @@ def simulateBatch(openDusts, deviceIndex="0", useGraph=True, alphas=None, precis
     until the longest simulation ends; the extra steps of shorter ones are
     computed and discarded.  tune=True lets the autotuner pick the pair
     kernel's schedule and tile shape (od_batch_tune); the choice
-    (sym_chunk, sym_tile) is returned, and results are reproducible for it
+    (sym_chunk, sym_tile), (0, 0) for the wave tiles, is returned, and results are reproducible for it
     (pass it back as sym_chunk and sym_tile).  progress(done, total) is called
     after every chunk of steps."""
     if len(openDusts) == 0:
