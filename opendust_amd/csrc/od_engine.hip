@@ -816,12 +816,16 @@ static double cell_list_units(const od_config* cfg, int n, CellGrid g) {
 // 5.4), FP32c 32768 ions 0.24 -> 0.06, 262144 1.07 -> 0.55, 2^20 5.6 -> 5.0
 // (with the pairs out of range skipped and cl_waves 0.39, 0.05, 0.46 and 3.8);
 // at 2^22 the choice is columns of cutoff/4.
+// Grids of more cells than half the ions (or 65536) are left out: false if none
+// remains, where the ions are so thin that most cells are empty whatever the
+// grid, entries outnumber ions many times, and the older kernels are faster
+// (16384 ions, r_c = 1 in R = 20, H = 80: 0.78 ms per step and 1.6 GB with the
+// list on columns of cutoff/4, 0.64 ms and 0.2 GB without; FP64 0.87 and 0.43).
 constexpr double CELL_ENTRY_COST = 24.0;
-static CellGrid choose_grid(const od_config* cfg, int n) {
+static bool choose_grid(const od_config* cfg, int n, CellGrid* best) {
   static const int qs[] = {8, 16, 32};
   const double pi = 3.141592653589793;
   const double dens = n / (pi * cfg->R * cfg->R * cfg->H);
-  CellGrid best;
   double best_cost = 1e300;
   for (int p2 = 1; p2 <= 10; ++p2) {
     const double w = 2.0 * cfg->cutoff / p2, nxd = ceil(2.0 * cfg->R / w);
@@ -860,25 +864,26 @@ static CellGrid choose_grid(const od_config* cfg, int n) {
       if (bulk) cost *= pi * cfg->R * cfg->R / (w * w);
       if (cost < best_cost) {
         best_cost = cost;
-        best = g;
+        *best = g;
       }
     }
   }
-  return best;
+  return best_cost < 1e300;
 }
 
-// Whether the context runs k_cell_list: where its partials, at twice the even
-// spread's units, fit CELL_LIST_MAX_BYTES, unless the configuration fixes a
-// variant of k_pair32_symcol.
+// Whether the context runs k_cell_list, and its grid: where choose_grid has one
+// and the partials, at twice the even spread's units, fit CELL_LIST_MAX_BYTES,
+// unless the configuration fixes a variant of k_pair32_symcol.
 constexpr double CELL_LIST_MAX_BYTES = 24e9;
 // below COUNT_MAX, so a unit count that saturated is over every capacity
 constexpr int CELL_LIST_MAX_UNITS = 1000000000;
 static_assert(CELL_LIST_MAX_UNITS < COUNT_MAX, "a saturated unit count must exceed the capacity");
-static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, CellGrid g, int* cap) {
-  const double units = 2.0 * cell_list_units(cfg, c->n, g) + 4096.0;
+static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, CellGrid* g, int* cap) {
   const bool fp32 = c->prec == OD_PREC_FP32C;
-  *cap = (int)std::min(units, (double)CELL_LIST_MAX_UNITS);
   if (fp32 && cfg->sym_tile > 0) return false;
+  if (!choose_grid(cfg, c->n, g)) return false;
+  const double units = 2.0 * cell_list_units(cfg, c->n, *g) + 4096.0;
+  *cap = (int)std::min(units, (double)CELL_LIST_MAX_UNITS);
   return units * 192.0 * (fp32 ? 4.0 : 8.0) <= CELL_LIST_MAX_BYTES;
 }
 
@@ -890,8 +895,8 @@ static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
     return set_err(OD_ERR_ARG, "cutoff %g nm in a cylinder R = %g, H = %g nm gives more than %d cells", cfg->cutoff,
                    cfg->R, cfg->H, OD_MAX_CELLS);
   c->cut = 1;
-  const CellGrid g = choose_grid(cfg, c->n);
-  c->list = cell_list_chosen(c, cfg, g, &c->cl_cap) ? 1 : 0;
+  CellGrid g;
+  c->list = cell_list_chosen(c, cfg, &g, &c->cl_cap) ? 1 : 0;
   if (c->list) {
     c->grid = g;
     fill_params(cfg, c->n_pad, &hp, g);

@@ -28,27 +28,35 @@ def say(*a):
     print(*a, flush=True)
 
 
-@contextlib.contextmanager
-def gpu_memory_left(left):
-    """Holds all device memory but `left` bytes (allocated, never touched)."""
+def _hip():
+    """The HIP runtime that the engine library is linked to."""
     from opendust_amd import engine
 
     engine.load_library()
     with open("/proc/self/maps") as f:
-        path = next(w.split()[-1] for w in f if "libamdhip64" in w)
-    hip = ctypes.CDLL(path)
+        return ctypes.CDLL(next(w.split()[-1] for w in f if "libamdhip64" in w))
+
+
+def gpu_free_bytes():
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@contextlib.contextmanager
+def gpu_memory_left(left):
+    """Holds all device memory but `left` bytes (allocated, never touched)."""
+    hip = _hip()
     held = []
     try:
         while True:
-            assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-            take = min(free.value - left, 32 << 30)
+            take = min(gpu_free_bytes() - left, 32 << 30)
             if take < 1 << 20:
                 break
             p = ctypes.c_void_p()
             assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(take)) == 0
             held.append(p)
-        say("  device memory left, GB:", round(free.value / 1e9, 2))
+        say("  device memory left, GB:", round(gpu_free_bytes() / 1e9, 2))
         yield
     finally:
         for p in held:

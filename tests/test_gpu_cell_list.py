@@ -8,7 +8,7 @@ import io
 import numpy as np
 import pytest
 
-from conftest import say
+from conftest import gpu_free_bytes, say
 
 pytestmark = pytest.mark.gpu
 
@@ -64,6 +64,26 @@ def _check(oracle_lib, cfg, x0, precision):
 def test_cell_list_sizes_vs_oracle(oracle_lib, precision, N, rc, rs):
     cfg, x0, _ = _setup(N, precision, rc, rs)
     say("cell list", precision, "N", N, "rc", rc, "rs", rs)
+    _check(oracle_lib, cfg, x0, precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+def test_sparse_cylinder_keeps_the_older_kernels(oracle_lib, precision):
+    """So few ions per cutoff that every grid of the list has more cells than
+    half the ions: the older kernels on columns of cutoff/4, whose memory is
+    the cells' (33 million) and not the list's entries'."""
+    from opendust_amd import engine
+
+    cfg, x0, _ = _setup(16384, precision, 1.0, None, R=20.0, H=80.0)
+    say("sparse cylinder", precision)
+    before = gpu_free_bytes()
+    e = engine.Engine(cfg)
+    held = before - gpu_free_bytes()
+    say("  device memory of the context, GB:", held / 1e9)
+    assert held <= 0.4e9
+    if precision == "fp32c":
+        assert e.sym_choice() == (0, 5)
+    e.close()
     _check(oracle_lib, cfg, x0, precision)
 
 
