@@ -171,7 +171,10 @@ typedef struct od_dust_record {
 typedef struct od_ctx od_ctx;
 
 /* Replaces mm.Context(system, integrator, platform, properties)
- * (opendust.py:1039-1042): allocates device state for cfg->n_ions ions. */
+ * (opendust.py:1039-1042): allocates device state for cfg->n_ions ions.  The
+ * automatic kernels with large partial sums (wave tiles, up to 48 GB; the evenly
+ * split cell list, up to 24 GB) are taken where they fit the free device memory,
+ * else the older kernels. */
 int od_create(const od_config* cfg, od_ctx** out);
 
 /* Replaces context.setPositions / setVelocities (opendust.py:1043-1044).

@@ -488,6 +488,9 @@ static int fill_params(const od_config* c, int n_pad, DevParams* P, CellGrid gri
   return OD_OK;
 }
 
+static void free_tile(TilePlan* t);
+static void free_cells(od_ctx* c);
+
 static void free_ctx(od_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->dev);  // teardown: nothing to report a failure to
@@ -496,11 +499,11 @@ static void free_ctx(od_ctx* c) {
   void* bufs[] = {c->dP, c->X, c->V, c->F, c->Fpart, c->q, c->partials, c->rowF, c->pi, c->pj,
                   c->list_old, c->list_new, c->flags, c->st, c->face, c->block_cnt, c->block_off, c->n_flag,
                   c->slot_of, c->list_ion, c->err, c->rec, c->wg_tab, c->wg_base, c->sym_tp, c->sym_dg,
-                  c->rowD, c->sym_sp, c->sym_acc, c->Gcut, c->scan_tsum, c->scan_toff, c->sc_tp, c->sc_sp, c->ckey[0], c->ckey[1], c->cval[0], c->cval[1], c->rs_hist,
-                  c->rs_off, c->rs_total, c->cell_start, c->cell_chunks, c->item_off, c->items,
-                  c->n_items, c->spos, c->tl.subs, c->tl.tp, c->cl_rng, c->cl_tp, c->rc4_cell};
+                  c->rowD, c->sym_sp, c->sym_acc};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  free_tile(&c->tl);
+  free_cells(c);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   for (hipEvent_t e : c->kev)
@@ -517,7 +520,28 @@ static int dalloc(P** p, size_t bytes) {
   return OD_OK;
 }
 
-// Builds the wave-tile plan *t (once per context).
+// Wave tiles and the evenly split cell list keep partial sums that grow with
+// the square of the density, where the older kernels hold little.  A context
+// takes them only if they fit and leave the device this much for what its
+// other calls allocate (od_pair_forces: up to 112 bytes per ion) and for the
+// runtime; else it steps down to the older kernels.
+static bool memory_left(int64_t n_ions) {
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return (double)free_b >= 128.0 * (double)n_ions + 256e6;
+}
+
+static void free_tile(TilePlan* t) {
+  if (t->subs) (void)hipFree(t->subs);
+  if (t->tp) (void)hipFree(t->tp);
+  *t = TilePlan();
+}
+
+// Builds the wave-tile plan *t (once per context); OD_ERR_HIP and an empty plan
+// if the memory is short.
 static int tile_build(TilePlan* t, const TileSims& sims, bool fp32) {
   *t = TilePlan();
   tile_shape(sims, fp32, &t->mt, &t->nw);
@@ -556,14 +580,21 @@ static int tile_build(TilePlan* t, const TileSims& sims, bool fp32) {
   std::memcpy(tab.data() + b_sub + b_grp, wg.data(), b_wg);
   char *d_tab = nullptr, *d_sum = nullptr;
   const size_t b_tp = segs * 192 * gm * 8;
-  CHKRET(dalloc(&d_tab, tab.size()));
+  int rc = dalloc(&d_tab, tab.size());
+  if (rc == OD_OK) rc = dalloc(&d_sum, b_tp + (size_t)u * 192 * (fp32 ? 4 : 8));
   t->subs = (int4*)d_tab;
+  t->tp = (double*)d_sum;
+  if (rc == OD_OK && !memory_left((int64_t)t->n_sub * 64))
+    rc = set_err(OD_ERR_HIP, "wave tiles: too little device memory left");
+  if (rc == OD_OK && hipMemcpy(d_tab, tab.data(), tab.size(), hipMemcpyHostToDevice) != hipSuccess)
+    rc = set_err(OD_ERR_HIP, "wave tiles: upload failed");
+  if (rc != OD_OK) {
+    free_tile(t);
+    return rc;
+  }
   t->groups = (TileGroup*)(d_tab + b_sub);
   t->wg_group = (int*)(d_tab + b_sub + b_grp);
-  CHKRET(dalloc(&d_sum, b_tp + (size_t)u * 192 * (fp32 ? 4 : 8)));
-  t->tp = (double*)d_sum;
   t->sp = d_sum + b_tp;
-  HIPCHK(hipMemcpy(d_tab, tab.data(), tab.size(), hipMemcpyHostToDevice));
   return OD_OK;
 }
 
@@ -887,20 +918,8 @@ static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, CellGrid* g,
   return units * 192.0 * (fp32 ? 4.0 : 8.0) <= CELL_LIST_MAX_BYTES;
 }
 
-// hp: the parameters with od_get_cells' grid; gets the context's own
-static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
-  c->cut = 0;
-  if (!(cfg->cutoff > 0.0)) return OD_OK;
-  if (hp.rc4_cells < 0)
-    return set_err(OD_ERR_ARG, "cutoff %g nm in a cylinder R = %g, H = %g nm gives more than %d cells", cfg->cutoff,
-                   cfg->R, cfg->H, OD_MAX_CELLS);
-  c->cut = 1;
-  CellGrid g;
-  c->list = cell_list_chosen(c, cfg, &g, &c->cl_cap) ? 1 : 0;
-  if (c->list) {
-    c->grid = g;
-    fill_params(cfg, c->n_pad, &hp, g);
-  }
+// the cell list's buffers on hp's grid (c->list: with those of k_cell_list)
+static int alloc_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   c->n_set = hp.n_fwd + 1;
   c->n_cells = hp.n_cells;
   c->n_cols = hp.nx * hp.ny;
@@ -953,6 +972,42 @@ static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
   return OD_OK;
 }
 
+static void free_cells(od_ctx* c) {
+  void** bufs[] = {(void**)&c->ckey[0], (void**)&c->ckey[1], (void**)&c->cval[0], (void**)&c->cval[1],
+                   (void**)&c->rs_hist, (void**)&c->rs_off, (void**)&c->rs_total, (void**)&c->cell_start,
+                   (void**)&c->cell_chunks, (void**)&c->item_off, (void**)&c->items, (void**)&c->n_items,
+                   (void**)&c->spos, (void**)&c->Gcut, (void**)&c->scan_tsum, (void**)&c->scan_toff,
+                   (void**)&c->cl_rng, (void**)&c->rc4_cell, (void**)&c->cl_tp, (void**)&c->sc_tp, (void**)&c->sc_sp};
+  for (void** b : bufs) {
+    if (*b) (void)hipFree(*b);
+    *b = nullptr;
+  }
+}
+
+// hp: the parameters with od_get_cells' grid; gets the context's own
+static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
+  c->cut = 0;
+  if (!(cfg->cutoff > 0.0)) return OD_OK;
+  if (hp.rc4_cells < 0)
+    return set_err(OD_ERR_ARG, "cutoff %g nm in a cylinder R = %g, H = %g nm gives more than %d cells", cfg->cutoff,
+                   cfg->R, cfg->H, OD_MAX_CELLS);
+  c->cut = 1;
+  CellGrid g;
+  c->list = cell_list_chosen(c, cfg, &g, &c->cl_cap) ? 1 : 0;
+  if (c->list) {
+    c->grid = g;
+    fill_params(cfg, c->n_pad, &hp, g);
+    const int rc = alloc_cells(c, cfg, hp);
+    if (rc != OD_ERR_HIP && (rc != OD_OK || memory_left(c->n_pad))) return rc;
+    // the memory is short: the older kernels, on their own grid
+    free_cells(c);
+    c->list = 0;
+    c->grid = CellGrid();
+    fill_params(cfg, c->n_pad, &hp);
+  }
+  return alloc_cells(c, cfg, hp);
+}
+
 // Whether a configuration without a schedule of its own runs the wave tiles:
 // FP64 whenever their partials fit; FP32 below TILE_FP32_SUBS sub-blocks of
 // 64 ions per simulation, above which the row groups of k_pair32_sym are
@@ -982,9 +1037,9 @@ static int setup_sym(od_ctx* c, const od_config* cfg) {
   c->tile = 0;
   const TileSims sims = ctx_sims(c);
   if (tile_chosen(cfg, sims)) {
-    CHKRET(tile_build(&c->tl, sims, c->prec == OD_PREC_FP32C));
-    c->tile = 1;
-    return OD_OK;
+    const int rc = tile_build(&c->tl, sims, c->prec == OD_PREC_FP32C);
+    c->tile = rc == OD_OK;
+    if (rc != OD_ERR_HIP) return rc;
   }
   return setup_k_pair32_sym(c, cfg);
 }

@@ -8,7 +8,7 @@ import io
 import numpy as np
 import pytest
 
-from conftest import gpu_free_bytes, say
+from conftest import gpu_free_bytes, gpu_memory_left, say
 
 pytestmark = pytest.mark.gpu
 
@@ -85,6 +85,37 @@ def test_sparse_cylinder_keeps_the_older_kernels(oracle_lib, precision):
         assert e.sym_choice() == (0, 5)
     e.close()
     _check(oracle_lib, cfg, x0, precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+def test_short_memory_steps_down_to_the_older_kernels(precision):
+    """2^20 ions at r_c = 2 in R = 10, H = 20 on a GPU with less free memory
+    than the list wants: the older kernels on their own grid, the same forces
+    up to rounding (FP32c: and up to pairs at the cutoff counted on one side,
+    each one pair force there)."""
+    from opendust_amd import engine
+
+    cfg, x0, _ = _setup(1 << 20, precision, 2.0, None, R=10.0, H=20.0)
+    say("short memory, cutoff", precision)
+    before = gpu_free_bytes()
+    e = engine.Engine(cfg)
+    held = before - gpu_free_bytes()
+    say("  device memory of the context, GB:", held / 1e9)
+    f = e.pair_forces(x0)
+    assert e.sym_choice() == (0, 0)
+    e.close()
+    assert held >= 3e9
+    with gpu_memory_left(int(held - 0.7e9)):
+        e = engine.Engine(cfg)
+        g = e.pair_forces(x0)
+        choice = e.sym_choice()
+        e.close()
+    if precision == "fp64":
+        fn = np.linalg.norm(f, axis=1)
+        assert np.all(np.linalg.norm(g - f, axis=1) <= 1e-11 * fn + 1e-13 * np.sqrt(np.mean(fn ** 2)))
+    else:
+        assert choice == (0, 5)
+        assert np.linalg.norm(g - f) <= 1e-5 * np.linalg.norm(f)
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])

@@ -147,6 +147,56 @@ def test_batch_tune_out_of_memory_keeps_wave_tiles():
     b.close()
 
 
+def test_short_memory_steps_down_to_rows():
+    """2^19 ions in FP64 want 3.2 GB of partial sums: on a GPU with less free,
+    the row kernel, with the same forces."""
+    from opendust_amd import engine
+
+    cfg, x0, _ = _setup(1 << 19, "fp64")
+    say("short memory, FP64 context")
+    f, info = _forces(cfg, x0, engine.PAIR_AUTO)
+    assert info[0] == engine.PAIR_SYM
+    with gpu_memory_left(2500 << 20):
+        g, info = _forces(cfg, x0, engine.PAIR_AUTO)
+    assert info[0] == engine.PAIR_ROWS
+    fn = np.linalg.norm(f, axis=1)
+    assert np.all(np.linalg.norm(g - f, axis=1) <= 1e-11 * fn + 1e-13 * np.sqrt(np.mean(fn ** 2)))
+
+
+@pytest.mark.parametrize("precision,n_sims,left", [("fp64", 3, 2300), ("fp32c", 6, 5000)])
+def test_short_memory_batch_steps_down(precision, n_sims, left):
+    """Simulations of 2^18 ions whose wave tiles do not fit: FP64 the row
+    items, FP32c the block schedule (whose launch leaves out the pairs inside
+    a block), with the same step up to rounding."""
+    from opendust_amd import engine
+
+    cfg, x0, v0 = _setup(262080, precision)
+    cfgs = []
+    for s in range(n_sims):
+        cfgs.append(engine.Config.from_buffer_copy(cfg))
+        cfgs[s].sim_id = s
+
+    def step():
+        b = engine.Batch(cfgs)
+        for s in range(n_sims):
+            b.set_ions(s, x0, v0)
+        b.run(1)
+        x, v = b.get_ions(n_sims - 1)
+        pairs = b.pair_timing()[2]
+        b.close()
+        return x, v, pairs
+
+    say("short memory, batch", precision)
+    x, v, pairs = step()
+    with gpu_memory_left(left << 20):
+        xs, vs, pairs_s = step()
+    assert pairs == n_sims * 262080 * 262079
+    assert pairs_s == pairs if precision == "fp64" else pairs_s < pairs
+    tol = 1e-12 if precision == "fp64" else 1e-6
+    assert not np.array_equal(v, vs)  # another order of the sums
+    assert np.max(np.abs(x - xs)) <= tol * cfg.R and np.max(np.abs(v - vs)) <= tol * np.max(np.abs(v))
+
+
 def test_fp64_pair_law_over_its_range():
     """Two ions from 1e-6 to 600 r_D_e apart, FP64 (rsqrt, exp and 1/x of the
     kernels' own), against numpy: about 10 roundings, and the rounding of the
