@@ -335,6 +335,7 @@ struct od_ctx {
   // cutoff mode: cell list; Gcut: flagged sources' share of the drift-state force;
   // sc_tp, sc_sp: partials of the symmetric cell kernel (FP32c)
   double* Gcut = nullptr;
+  char* cell_sums = nullptr;  // holds the partial sums below
   double* sc_tp = nullptr;
   float* sc_sp = nullptr;
   int *scan_tsum = nullptr, *scan_toff = nullptr;
@@ -950,22 +951,29 @@ static int alloc_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   const size_t n_tiles = (n_scan + 1023) / 1024;
   if ((rc = dalloc(&c->scan_tsum, n_tiles * 4)) || (rc = dalloc(&c->scan_toff, n_tiles * 4))) return rc;
   c->sc_var = CC_DEFAULT;
+  const bool fp32 = c->prec == OD_PREC_FP32C;
+  const size_t b_sc = fp32 ? (size_t)c->n_set * 3 * np * 8 : 0;
+  const size_t b_tp = c->list ? ((size_t)cl_waves(c->n) + c->max_items) * 3 * CL_G * 8 : 0;
+  const size_t b_list = c->list ? b_tp + (size_t)c->cl_cap * 192 * (fp32 ? 4 : 8) : 0;
   if (c->list) {
-    // one allocation for the tables, one for the partial sums
+    // one allocation for the tables
     const size_t ne = (size_t)c->n_entries + 1;
-    const size_t b_tp = ((size_t)cl_waves(c->n) + c->max_items) * 3 * CL_G * 8;
-    if ((rc = dalloc(&c->cl_rng, ne * 16 + 4)) || (rc = dalloc(&c->rc4_cell, np * 4)) ||
-        (rc = dalloc(&c->cl_tp, b_tp + (size_t)c->cl_cap * 192 * (c->prec == OD_PREC_FP32C ? 4 : 8))))
-      return rc;
+    if ((rc = dalloc(&c->cl_rng, ne * 16 + 4)) || (rc = dalloc(&c->rc4_cell, np * 4))) return rc;
     c->cl_cnt = (int*)(c->cl_rng + ne);
     c->cl_u0 = c->cl_cnt + ne;
     c->cl_total = c->cl_u0 + ne;
-    c->cl_sp = (char*)c->cl_tp + b_tp;
   }
-  if (c->prec == OD_PREC_FP32C) {
-    if ((rc = dalloc(&c->sc_tp, (size_t)c->n_set * 3 * np * 8)) ||
-        (rc = dalloc(&c->sc_sp, (size_t)c->n_set * 3 * np * 4)))
-      return rc;
+  // one for the partial sums: an evaluation writes either the list's or, where
+  // that has no room, k_pair32_symcol's, so both lie in the same place (2^22
+  // ions: 23.7 GB instead of 29.6)
+  if ((b_list || b_sc) && (rc = dalloc(&c->cell_sums, std::max(b_list, b_sc + b_sc / 2)))) return rc;
+  if (c->list) {
+    c->cl_tp = (double*)c->cell_sums;
+    c->cl_sp = c->cell_sums + b_tp;
+  }
+  if (fp32) {
+    c->sc_tp = (double*)c->cell_sums;
+    c->sc_sp = (float*)(c->cell_sums + b_sc);
     c->sc_var = cell_variant_of(cfg->sym_tile);
     if (c->sc_var < 0) return set_err(OD_ERR_ARG, "cutoff mode: sym_tile %d outside [0, %d]", cfg->sym_tile, CC_N_VARIANTS);
   }
@@ -977,7 +985,7 @@ static void free_cells(od_ctx* c) {
                    (void**)&c->rs_hist, (void**)&c->rs_off, (void**)&c->rs_total, (void**)&c->cell_start,
                    (void**)&c->cell_chunks, (void**)&c->item_off, (void**)&c->items, (void**)&c->n_items,
                    (void**)&c->spos, (void**)&c->Gcut, (void**)&c->scan_tsum, (void**)&c->scan_toff,
-                   (void**)&c->cl_rng, (void**)&c->rc4_cell, (void**)&c->cl_tp, (void**)&c->sc_tp, (void**)&c->sc_sp};
+                   (void**)&c->cl_rng, (void**)&c->rc4_cell, (void**)&c->cell_sums};
   for (void** b : bufs) {
     if (*b) (void)hipFree(*b);
     *b = nullptr;
@@ -2155,6 +2163,17 @@ static int tune_cells(od_ctx* c, int reps, int* chosen_var) {
   return rc;
 }
 
+// frees the schedule of k_pair32_sym and its partial sums (the stream is idle)
+static void release_sym(od_ctx* c) {
+  void* bufs[] = {c->wg_tab, c->wg_base, c->sym_tp, c->sym_sp, c->sym_dg, c->sym_acc};
+  for (void* q : bufs)
+    if (q) (void)hipFree(q);
+  c->wg_tab = nullptr;
+  c->wg_base = nullptr;
+  c->sym_tp = c->sym_dg = c->sym_acc = nullptr;
+  c->sym_sp = nullptr;
+}
+
 extern "C" int od_tune(od_ctx* c, int32_t reps, int32_t* sym_chunk, int32_t* sym_tile) {
   if (!c) return set_err(OD_ERR_ARG, "null context");
   if (reps < 1 || reps > 100) return set_err(OD_ERR_ARG, "reps %d outside [1, 100]", reps);
@@ -2189,6 +2208,8 @@ extern "C" int od_tune(od_ctx* c, int32_t reps, int32_t* sym_chunk, int32_t* sym
     if (rc == OD_OK) rc = tune_sym(c, be, reps, evaluate, &chosen, &var, c->band_cap, SYM_BAND_BYTES, &sym_ms);
     (void)hipFree(Fs);
     if (tiles && (rc != OD_OK || tile_ms <= sym_ms)) {
+      if (rc != OD_OK) (void)hipStreamSynchronize(c->stream);
+      release_sym(c);
       c->tile = 1;
       c->sym = 0;
       chosen = 0;

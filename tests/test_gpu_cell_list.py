@@ -104,7 +104,9 @@ def test_short_memory_steps_down_to_the_older_kernels(precision):
     f = e.pair_forces(x0)
     assert e.sym_choice() == (0, 0)
     e.close()
-    assert held >= 3e9
+    # beside the partial sums (FP64 4.8, FP32c 2.6 GB) under 0.3 kB per ion: the
+    # fallback kernel's lie in the same place
+    assert 2.5e9 <= held <= (5.2e9 if precision == "fp64" else 2.95e9)
     with gpu_memory_left(int(held - 0.7e9)):
         e = engine.Engine(cfg)
         g = e.pair_forces(x0)

@@ -7,7 +7,7 @@ import io
 import numpy as np
 import pytest
 
-from conftest import gpu_memory_left, say
+from conftest import gpu_free_bytes, gpu_memory_left, say
 
 pytestmark = pytest.mark.gpu
 
@@ -102,11 +102,13 @@ def test_tune_keeps_or_replaces_wave_tiles():
     e.set_ions(x0, v0)
     f0 = e.pair_forces(x0)
     say("tune over wave tiles")
+    before = gpu_free_bytes()
     chosen = e.tune(2)
     f1 = e.pair_forces(x0)
     assert e.sym_choice() == chosen
     if chosen == (0, 0):
         assert np.array_equal(f0, f1)
+        assert before - gpu_free_bytes() <= 2e6  # the schedules it timed are gone
     else:
         assert np.linalg.norm(f1 - f0) <= 4e-6 * np.linalg.norm(f0)
     e.run(4, engine.RUN_GRAPH)
