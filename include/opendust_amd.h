@@ -43,7 +43,7 @@ extern "C" {
 #define OD_DIST_FIELD_DRIVEN 1
 
 /* pair-force precision */
-#define OD_PREC_FP32C 0 /* FP32 pair arithmetic, compensated (Kahan) per-ion sums */
+#define OD_PREC_FP32C 0 /* FP32 pair arithmetic; per-ion sums of short FP32 chains, added compensated or in FP64 */
 #define OD_PREC_FP64 1  /* plain FP64 pair arithmetic */
 
 /* all-pairs kernel */

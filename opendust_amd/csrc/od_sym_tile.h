@@ -294,14 +294,16 @@ __device__ __forceinline__ float wave_ror1(float v) {
 // that the others needed.  Cutoff force evaluation at 2^22 ions 52.2 -> 44.5
 // ms, 2^20 4.9 -> 4.2 (with the compare on r2, which skips the square root).
 // ls: this lane's entry ls + lane + 64.  (bx, by, bz): added to.
+// sym_steps_lds: steps first .. last - 1 alone (a multiple of UN): afterwards
+// lane l holds the reaction of these steps on source (l - last) mod 64.
 template <int MT, int CUT, bool PF = false, int UN = 16>
-__device__ __forceinline__ void sym_tile_lds(SymT<MT>& T, const float4* ls, float& bx, float& by, float& bz,
-                                             const SymLaw& L) {
+__device__ __forceinline__ void sym_steps_lds(SymT<MT>& T, const float4* ls, int first, int last, float& bx,
+                                              float& by, float& bz, const SymLaw& L) {
   const float eps = vgpr(EPS32);
-  // PF: the read after the last step, ls[-64], is the lane's own entry
-  // ls[lane] (in bounds, unused)
-  float4 qn = ls[0];
-  for (int s0 = 0; s0 < 64; s0 += UN) {
+  // PF: the read after the last step, ls[-last], is another lane's source or,
+  // at -64, the lane's own entry ls[lane] (in bounds, unused)
+  float4 qn = ls[-first];
+  for (int s0 = first; s0 < last; s0 += UN) {
 #pragma unroll
     for (int s = 0; s < UN; ++s) {
       float4 q;
@@ -356,6 +358,12 @@ __device__ __forceinline__ void sym_tile_lds(SymT<MT>& T, const float4* ls, floa
       }
     }
   }
+}
+
+template <int MT, int CUT, bool PF = false, int UN = 16>
+__device__ __forceinline__ void sym_tile_lds(SymT<MT>& T, const float4* ls, float& bx, float& by, float& bz,
+                                             const SymLaw& L) {
+  sym_steps_lds<MT, CUT, PF, UN>(T, ls, 0, 64, bx, by, bz, L);
 }
 
 // The 64 x 64 pairs of the wave's source sub-block (xj, yj, zj, one per lane)

@@ -63,6 +63,30 @@ def test_wave_tiles_vs_oracle_or_rows(oracle_lib, precision, N):
     assert np.linalg.norm(f - ref) <= rel * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("N", [2000, 8000, 32704, 65536])
+def test_wave_tiles_round_no_worse_than_rows(N):
+    """FP32c forces of the wave tiles and of the row kernel, which adds
+    compensated 64-term blocks, against FP64 on the positions both see: the
+    tiles' median error per ion is not larger (5 % for the spread of a median
+    over N ions)."""
+    from oracle.oracle import fp32c_rounded_positions
+
+    from opendust_amd import engine, host
+
+    cfg, x0, _ = _setup(N, "fp32c")
+    cfg64 = engine.Config.from_buffer_copy(cfg)
+    cfg64.precision = host.PREC_FP64
+    say("rounding of wave tiles, N", N)
+    ref, _ = _forces(cfg64, fp32c_rounded_positions(cfg, x0), engine.PAIR_AUTO)
+    fn = np.linalg.norm(ref, axis=1)
+    err = {}
+    for mode in (engine.PAIR_AUTO, engine.PAIR_ROWS):
+        f, _ = _forces(cfg, x0, mode)
+        err[mode] = float(np.median(np.linalg.norm(f - ref, axis=1) / fn))
+    say("  median error per ion, tiles and rows:", err[engine.PAIR_AUTO], err[engine.PAIR_ROWS])
+    assert err[engine.PAIR_AUTO] <= 1.05 * err[engine.PAIR_ROWS]
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 def test_wave_tiles_batch_equals_single(precision):
     """Simulations of a batch whose sizes end inside a sub-block and a group:
