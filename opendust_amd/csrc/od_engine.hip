@@ -349,7 +349,7 @@ struct od_ctx {
   int2* items = nullptr;
   void* spos = nullptr;
   // even split of the cell list (k_cell_list): entries, first units, partials
-  int list = 0, cl_cap = 0, n_entries = 0, item_len = 64;
+  int list = 0, cl_cap = 0, n_entries = 0, item_len = 64, cl_chain = 64;
   CellGrid grid;
   int n_set = 0;                  // forward column offsets + 1
   uint32_t* rc4_cell = nullptr;   // od_get_cells' cells, where the grid is another
@@ -903,6 +903,22 @@ static bool choose_grid(const od_config* cfg, int n, CellGrid* best) {
   return best_cost < 1e300;
 }
 
+// FP32 chain length of k_cell_list (CH).  Its wide columns fill a 64-source
+// unit with pairs in range, where a column of cutoff/4, which the older kernels
+// run on, holds a few ions within the cutoff (`window`) and so adds up short
+// chains; chains are kept about as short.  Median error per ion against 64 bits
+// (positions rounded to FP32, r_c = 2, R = 10, H = 20): 32768 ions older kernels
+// 0.95e-7, one chain per unit 1.73e-7, now 0.90; 130001 1.31, 2.29, 1.14; 2^18 1.69,
+// 2.41, 1.13; 2^20 2.68, 2.93, 1.57; from 2^21 ions one chain is level (3.05, 3.07).
+// Step, one chain -> now: 2^15 ions 163 -> 169 us, 2^17 282 -> 292, 2^18 605 -> 627,
+// 2^20 4.19 -> 4.25 ms.
+static int chain_steps(const od_config* cfg, int n) {
+  const double pi = 3.141592653589793;
+  const double w = cfg->cutoff / 4.0;
+  const double window = n / (pi * cfg->R * cfg->R * cfg->H) * w * w * 2.0 * cfg->cutoff;
+  return window < 16.0 ? 4 : window < 48.0 ? 16 : window < 350.0 ? 32 : 64;
+}
+
 // Whether the context runs k_cell_list, and its grid: where choose_grid has one
 // and the partials, at twice the even spread's units, fit CELL_LIST_MAX_BYTES,
 // unless the configuration fixes a variant of k_pair32_symcol.
@@ -1004,6 +1020,7 @@ static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
   c->list = cell_list_chosen(c, cfg, &g, &c->cl_cap) ? 1 : 0;
   if (c->list) {
     c->grid = g;
+    c->cl_chain = chain_steps(cfg, c->n);
     fill_params(cfg, c->n_pad, &hp, g);
     const int rc = alloc_cells(c, cfg, hp);
     if (rc != OD_ERR_HIP && (rc != OD_OK || memory_left(c->n_pad))) return rc;
@@ -1344,8 +1361,13 @@ static int launch_forces_t(od_ctx* c, const double* X, const void* pos, const ui
   const int* n_units = c->list ? c->cl_total : nullptr;
   if (c->list) {
     // the kernels after these two return at once unless the units overflow
-    hipLaunchKernelGGL((sw ? k_cell_list<T, 2> : k_cell_list<T, 1>), dim3(cl_waves(c->n)), dim3(64), 0, c->stream,
-                       c->dP, (const PV*)c->spos, c->skey, c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries,
+    auto fn = sw ? k_cell_list<T, 2, 64> : k_cell_list<T, 1, 64>;
+    if constexpr (std::is_same<T, float>::value) {
+      if (c->cl_chain == 32) fn = sw ? k_cell_list<T, 2, 32> : k_cell_list<T, 1, 32>;
+      if (c->cl_chain == 16) fn = sw ? k_cell_list<T, 2, 16> : k_cell_list<T, 1, 16>;
+      if (c->cl_chain == 4) fn = sw ? k_cell_list<T, 2, 4> : k_cell_list<T, 1, 4>;
+    }
+    hipLaunchKernelGGL(fn, dim3(cl_waves(c->n)), dim3(64), 0, c->stream, c->dP, (const PV*)c->spos, c->skey, c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries,
                        n_units, c->cl_cap, c->cl_tp, (T*)c->cl_sp);
     hipLaunchKernelGGL(k_cell_list_reduce<T>, dim3(c->n_pad / 64), dim3(64 * REDUCE_PARTS), 0, c->stream, c->dP,
                        c->skey, c->sval, c->cell_start, c->item_off, c->cl_rng, c->cl_u0, n_units, c->cl_cap, cl_waves(c->n),

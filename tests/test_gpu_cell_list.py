@@ -120,6 +120,36 @@ def test_short_memory_steps_down_to_the_older_kernels(precision):
         assert np.linalg.norm(g - f) <= 1e-5 * np.linalg.norm(f)
 
 
+@pytest.mark.parametrize("N,R,H,rc,rs", [(32768, 10.0, 20.0, 2.0, None), (60000, 10.0, 20.0, 2.0, None),
+                                         (130001, 10.0, 20.0, 2.0, None), (310000, 10.0, 20.0, 2.0, None),
+                                         (20000, 3.0, 6.0, 3.2, 3.0), (4000, 3.0, 6.0, 3.2, 3.0)])
+def test_cell_list_rounds_no_worse_than_the_older_kernels(N, R, H, rc, rs):
+    """FP32c forces of the list and of the kernel on columns of cutoff/4
+    (sym_tile = 5), against FP64 on the positions both see, one size for each
+    length of the list's FP32 chains: its median error per ion is not larger
+    (5 % for the spread of a median over N ions)."""
+    from opendust_amd import engine, host
+    from oracle.oracle import fp32c_rounded_positions
+
+    cfg, x0, _ = _setup(N, "fp32c", rc, rs, R=R, H=H)
+    cfg64 = engine.Config.from_buffer_copy(cfg)
+    cfg64.precision = host.PREC_FP64
+    say("rounding of the cell list, N", N)
+    e = engine.Engine(cfg64)
+    ref = e.pair_forces(fp32c_rounded_positions(cfg, x0))
+    e.close()
+    fn = np.linalg.norm(ref, axis=1)
+    err = {}
+    for tile in (0, 5):
+        cfg.sym_tile = tile
+        e = engine.Engine(cfg)
+        err[tile] = float(np.median(np.linalg.norm(e.pair_forces(x0) - ref, axis=1)[fn > 0] / fn[fn > 0]))
+        assert e.sym_choice() == (0, tile)
+        e.close()
+    say("  median error per ion, list and older kernel:", err[0], err[5])
+    assert err[0] <= 1.05 * err[5]
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 @pytest.mark.parametrize("shape", ["cluster", "two_slabs", "line"])
 def test_cell_list_uneven_ions_vs_oracle(oracle_lib, precision, shape):
