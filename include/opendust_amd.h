@@ -282,12 +282,24 @@ int od_sym_variants(void);
 int od_sym_variant_info(int32_t v, int32_t* targets_per_lane, int32_t* waves_per_simd, int32_t* vgpr_operands,
                         int32_t* target_blocks);
 
-/* Cutoff mode only: the cell list of the last force evaluation.  cell_of_ion[n]
- * (binned ions: their cell; ions left out: the number of cells), sorted_ions
- * (binned ions in cell order, ties by ion index), their count, and the grid
- * dims[3].  Any pointer may be NULL.  No counterpart in the reference (OpenMM
- * keeps its neighbour list internal). */
+/* Cutoff mode only: the ions of the last force evaluation in the grid of columns
+ * cutoff/4 and slabs cutoff/16 (the evenly split cell list bins into another,
+ * od_get_force_cells).  cell_of_ion[n] (binned ions: their cell; ions left out:
+ * the number of cells), sorted_ions (binned ions in cell order, ties by ion
+ * index), their count, and the grid dims[3].  Any pointer may be NULL.  No
+ * counterpart in the reference (OpenMM keeps its neighbour list internal). */
 int od_get_cells(od_ctx* ctx, int32_t* cell_of_ion, int32_t* sorted_ions, int64_t* n_binned, int32_t* dims);
+
+/* Cutoff mode only (measurement support): the list that the forces of the last
+ * evaluation ran on, as the device sorted it: cell_of_ion, sorted_ions, n_binned
+ * and dims as in od_get_cells, on the forces' own grid; size[2]: its column
+ * width and slab height, nm (cell = iz + dims[2] (ix + dims[0] iy), with ix =
+ * floor((x + R) / size[0]), iz = floor((z + H/2) / size[1]), clamped to the
+ * grid); radix_passes of the sort; units and unit_capacity of the evenly split
+ * list (0 and 0: the context runs the older kernels; more units than capacity:
+ * they computed that evaluation's forces).  Any pointer may be NULL. */
+int od_get_force_cells(od_ctx* ctx, int32_t* cell_of_ion, int32_t* sorted_ions, int64_t* n_binned, int32_t* dims,
+                       double* size, int32_t* radix_passes, int64_t* units, int64_t* unit_capacity);
 
 /* Cutoff mode only, for the current cell list (measurement support):
  * ordered ion pairs within the cutoff, and the ordered pair terms the cell

@@ -1713,29 +1713,9 @@ extern "C" int od_run(od_ctx* c, int64_t nsteps, od_dust_record* out, int32_t fl
   return OD_OK;
 }
 
-extern "C" int od_get_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sorted_ions, int64_t* n_binned,
-                            int32_t* dims) {
-  if (!c) return set_err(OD_ERR_ARG, "null context");
-  if (!c->cut) return set_err(OD_ERR_STATE, "od_get_cells: context has no cutoff (no cell list)");
-  HIPCHK(hipSetDevice(c->dev));
-  std::vector<uint32_t> key(c->n_pad), val(c->n_pad);
-  DevParams hp;
-  fill_params(&c->cfg, c->n_pad, &hp);
-  const uint32_t n_cells = (uint32_t)hp.rc4_cells;
-  if (c->rc4_cell) {
-    // the forces' grid is another: (cell, ion) order of the binned ions
-    HIPCHK(hipMemcpyAsync(key.data(), c->rc4_cell, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    for (int i = 0; i < c->n_pad; ++i) val[i] = (uint32_t)i;
-    std::stable_sort(val.begin(), val.end(), [&](uint32_t a, uint32_t b) { return key[a] < key[b]; });
-    std::vector<uint32_t> sorted(c->n_pad);
-    for (int p = 0; p < c->n_pad; ++p) sorted[p] = std::min(key[val[p]], n_cells);
-    key.swap(sorted);
-  } else {
-    HIPCHK(hipMemcpyAsync(key.data(), c->skey, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(val.data(), c->sval, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-  }
+// cell ids and order of a sorted list (key, val), as od_get_cells reports them
+static int64_t report_cells(const od_ctx* c, const std::vector<uint32_t>& key, const std::vector<uint32_t>& val,
+                            uint32_t n_cells, int32_t* cell_of_ion, int32_t* sorted_ions) {
   int64_t nb = 0;
   for (int p = 0; p < c->n_pad; ++p) {
     const uint32_t i = val[p];
@@ -1745,12 +1725,77 @@ extern "C" int od_get_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sorted_ion
       ++nb;
     }
   }
+  return nb;
+}
+
+// the device's sorted list, and the units of its last evaluation
+static int download_list(od_ctx* c, std::vector<uint32_t>* key, std::vector<uint32_t>* val, int* units) {
+  key->resize(c->n_pad);
+  val->resize(c->n_pad);
+  HIPCHK(hipMemcpyAsync(key->data(), c->skey, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipMemcpyAsync(val->data(), c->sval, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
+  if (units && c->list) HIPCHK(hipMemcpyAsync(units, c->cl_total, 4, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
+  return OD_OK;
+}
+
+extern "C" int od_get_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sorted_ions, int64_t* n_binned,
+                            int32_t* dims) {
+  if (!c) return set_err(OD_ERR_ARG, "null context");
+  if (!c->cut) return set_err(OD_ERR_STATE, "od_get_cells: context has no cutoff (no cell list)");
+  HIPCHK(hipSetDevice(c->dev));
+  std::vector<uint32_t> key, val;
+  DevParams hp;
+  fill_params(&c->cfg, c->n_pad, &hp);
+  const uint32_t n_cells = (uint32_t)hp.rc4_cells;
+  if (c->rc4_cell) {
+    // the forces' grid is another: (cell, ion) order of the binned ions
+    std::vector<uint32_t> cell(c->n_pad);
+    HIPCHK(hipMemcpyAsync(cell.data(), c->rc4_cell, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    val.resize(c->n_pad);
+    for (int i = 0; i < c->n_pad; ++i) val[i] = (uint32_t)i;
+    std::stable_sort(val.begin(), val.end(), [&](uint32_t a, uint32_t b) { return cell[a] < cell[b]; });
+    key.resize(c->n_pad);
+    for (int p = 0; p < c->n_pad; ++p) key[p] = std::min(cell[val[p]], n_cells);
+  } else {
+    CHKRET(download_list(c, &key, &val, nullptr));
+  }
+  const int64_t nb = report_cells(c, key, val, n_cells, cell_of_ion, sorted_ions);
   if (n_binned) *n_binned = nb;
   if (dims) {
     dims[0] = hp.rc4_nx;
     dims[1] = hp.rc4_nx;
     dims[2] = hp.rc4_nz;
   }
+  return OD_OK;
+}
+
+extern "C" int od_get_force_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sorted_ions, int64_t* n_binned,
+                                  int32_t* dims, double* size, int32_t* radix_passes, int64_t* units,
+                                  int64_t* unit_capacity) {
+  if (!c) return set_err(OD_ERR_ARG, "null context");
+  if (!c->cut) return set_err(OD_ERR_STATE, "od_get_force_cells: context has no cutoff (no cell list)");
+  HIPCHK(hipSetDevice(c->dev));
+  std::vector<uint32_t> key, val;
+  int total = 0;
+  CHKRET(download_list(c, &key, &val, &total));
+  const int64_t nb = report_cells(c, key, val, (uint32_t)c->n_cells, cell_of_ion, sorted_ions);
+  if (n_binned) *n_binned = nb;
+  if (dims) {
+    dims[0] = c->nx;
+    dims[1] = c->ny;
+    dims[2] = c->nz;
+  }
+  if (size) {
+    DevParams hp;
+    fill_params(&c->cfg, c->n_pad, &hp, c->grid);
+    size[0] = hp.col_w;
+    size[1] = hp.slab_h;
+  }
+  if (radix_passes) *radix_passes = c->rs_passes;
+  if (units) *units = total;
+  if (unit_capacity) *unit_capacity = c->list ? c->cl_cap : 0;
   return OD_OK;
 }
 

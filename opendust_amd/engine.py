@@ -144,7 +144,7 @@ _lib = None
 EXPORTS = [
     "od_create", "od_set_ions", "od_get_ions", "od_set_dust_charges", "od_get_dust_charges",
     "od_set_step", "od_run", "od_pair_timing", "od_pair_info", "od_get_step_info", "od_pair_forces",
-    "od_get_cells", "od_cutoff_pair_count",
+    "od_get_cells", "od_get_force_cells", "od_cutoff_pair_count",
     "od_trap_potential_grid", "od_trap_samples_host", "od_abi_sizes", "od_destroy",
     "od_last_error", "od_build_info",
     "od_batch_create", "od_batch_set_ions", "od_batch_get_ions", "od_batch_run", "od_batch_get_step_info",
@@ -179,6 +179,9 @@ def load_library(path=LIB_PATH):
     lib.od_pair_info.argtypes = [c_ctx, P(ctypes.c_int32), P(ctypes.c_int64)]
     lib.od_stage_timing.argtypes = [c_ctx, dp, P(ctypes.c_int64), ctypes.c_int32]
     lib.od_get_cells.argtypes = [c_ctx, P(ctypes.c_int32), P(ctypes.c_int32), P(ctypes.c_int64), P(ctypes.c_int32)]
+    lib.od_get_force_cells.argtypes = [c_ctx, P(ctypes.c_int32), P(ctypes.c_int32), P(ctypes.c_int64),
+                                       P(ctypes.c_int32), dp, P(ctypes.c_int32), P(ctypes.c_int64),
+                                       P(ctypes.c_int64)]
     lib.od_cutoff_pair_count.argtypes = [c_ctx, P(ctypes.c_int64), P(ctypes.c_int64)]
     lib.od_get_step_info.argtypes = [c_ctx, P(ctypes.c_uint32), P(ctypes.c_uint8), P(ctypes.c_int64)]
     lib.od_pair_forces.argtypes = [c_ctx, dp, dp]
@@ -405,7 +408,8 @@ class Engine:
         return mode.value, pairs.value
 
     def cells(self):
-        """(cell_of_ion[n], sorted_ions[n_binned], dims) of the last cell list (cutoff mode)."""
+        """(cell_of_ion[n], sorted_ions[n_binned], dims) of the last force evaluation's ions in the
+        grid of columns cutoff/4, slabs cutoff/16 (cutoff mode)."""
         cell = np.empty(self.n, dtype=np.int32)
         order = np.empty(self.n, dtype=np.int32)
         nb = ctypes.c_int64()
@@ -414,6 +418,20 @@ class Engine:
         _check(self.lib.od_get_cells(self._ctx, cell.ctypes.data_as(i32), order.ctypes.data_as(i32),
                                      ctypes.byref(nb), dims), "od_get_cells")
         return cell, order[: nb.value], tuple(dims)
+
+    def force_cells(self):
+        """The list that the last cutoff forces ran on: dict of cell (per ion), order (sorted ions),
+        dims, size (column width, slab height, nm), radix_passes, units and capacity (od_get_force_cells)."""
+        cell = np.empty(self.n, dtype=np.int32)
+        order = np.empty(self.n, dtype=np.int32)
+        nb, units, cap = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
+        dims, size, passes = (ctypes.c_int32 * 3)(), (ctypes.c_double * 2)(), ctypes.c_int32()
+        i32 = ctypes.POINTER(ctypes.c_int32)
+        _check(self.lib.od_get_force_cells(self._ctx, cell.ctypes.data_as(i32), order.ctypes.data_as(i32),
+                                           ctypes.byref(nb), dims, size, ctypes.byref(passes), ctypes.byref(units),
+                                           ctypes.byref(cap)), "od_get_force_cells")
+        return {"cell": cell, "order": order[: nb.value], "dims": tuple(dims), "size": tuple(size),
+                "radix_passes": passes.value, "units": units.value, "capacity": cap.value}
 
     def cutoff_pair_count(self):
         a = ctypes.c_int64()

@@ -1,6 +1,7 @@
 """The even-split cell-list force (k_cell_list) where it can go wrong: few
 columns, groups and chunks that end inside a column, empty columns, clusters
-that overflow its buffer, and the grid it bins into."""
+that overflow its buffer, short memory, thin cylinders, the rounding of its
+sums, and the grid it bins into."""
 
 import contextlib
 import io
@@ -35,8 +36,20 @@ def _check(oracle_lib, cfg, x0, precision):
     e = engine.Engine(cfg)
     f = e.pair_forces(x0)
     cell, order, dims = e.cells()
+    fc = e.force_cells()
     f2 = e.pair_forces(x0)
     e.close()
+    # the device's own list: binning and radix order bit-exact on its grid
+    nx, ny, nz = fc["dims"]
+    w, h = fc["size"]
+    ix, iy = (np.clip(np.floor((x0[:, k] + cfg.R) / w), 0, nx - 1).astype(int) for k in (0, 1))
+    iz = np.clip(np.floor((x0[:, 2] + cfg.H / 2) / h), 0, nz - 1).astype(int)
+    want = iz + nz * (ix + nx * iy)
+    assert nx == ny == np.ceil(2 * cfg.R / w) and nz == np.ceil(cfg.H / h)
+    assert np.array_equal(fc["cell"], want)
+    assert np.array_equal(fc["order"], np.lexsort((np.arange(len(want)), want)))
+    assert 256 ** (fc["radix_passes"] - 1) <= max(1, nx * ny * nz) < 256 ** fc["radix_passes"]
+    say("  grid", fc["dims"], "radix passes", fc["radix_passes"], "units", fc["units"], "of", fc["capacity"])
     assert np.array_equal(f, f2)
     if precision == "fp64":
         ref, edge = oracle_lib.pair_forces(cfg, x0), np.zeros(len(x0))
@@ -56,6 +69,7 @@ def _check(oracle_lib, cfg, x0, precision):
     assert dims == oracle_lib.cell_of(cfg, x0[0])[1]
     assert np.array_equal(cell, want)
     assert np.array_equal(order, np.lexsort((np.arange(len(want)), want)))
+    return fc
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
@@ -84,7 +98,8 @@ def test_sparse_cylinder_keeps_the_older_kernels(oracle_lib, precision):
     if precision == "fp32c":
         assert e.sym_choice() == (0, 5)
     e.close()
-    _check(oracle_lib, cfg, x0, precision)
+    fc = _check(oracle_lib, cfg, x0, precision)
+    assert fc["capacity"] == 0 and fc["dims"] == (160, 160, 1280) and fc["radix_passes"] == 4
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
@@ -150,19 +165,25 @@ def test_cell_list_rounds_no_worse_than_the_older_kernels(N, R, H, rc, rs):
     assert err[0] <= 1.05 * err[5]
 
 
+def _ball(cfg, n, rng):
+    """n ions in a ball of half the cutoff, away from the dust"""
+    d = rng.normal(size=(n, 3))
+    r = 0.5 * cfg.cutoff * rng.uniform(size=n) ** (1 / 3)
+    return d / np.linalg.norm(d, axis=1)[:, None] * r[:, None] + [1.2 * cfg.r_D_e, 0.0, 3.0 * cfg.r_D_e]
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 @pytest.mark.parametrize("shape", ["cluster", "two_slabs", "line"])
 def test_cell_list_uneven_ions_vs_oracle(oracle_lib, precision, shape):
-    """Ions far from evenly spread.  cluster: all in a ball of half the cutoff
-    (every pair interacts; the units exceed the buffer, so the fallback
-    kernels compute the force); two_slabs: the middle of every column empty,
-    so a group spans the gap; line: one column holds everything."""
+    """Ions far from evenly spread, within the unit buffer.  cluster: all in a
+    ball of half the cutoff (every pair interacts); two_slabs: the middle of
+    every column empty, so a group spans the gap; line: one column holds
+    everything."""
     cfg, x0, _ = _setup(4000, precision, 1.0, None, R=3.0, H=30.0)
     rng = np.random.RandomState(5)
     lam = cfg.r_D_e
     if shape == "cluster":
-        d = rng.normal(size=x0.shape)
-        x0 = d / np.linalg.norm(d, axis=1)[:, None] * (0.5 * lam * rng.uniform(size=len(x0)) ** (1 / 3))[:, None]
+        x0 = _ball(cfg, len(x0), rng)
     elif shape == "two_slabs":
         x0[:, 2] = np.where(np.arange(len(x0)) % 2, 14.0, -14.0) * lam + rng.uniform(-0.4, 0.4, len(x0)) * lam
         x0[:50, 2] = rng.uniform(-14.0, 14.0, 50) * lam
@@ -170,4 +191,70 @@ def test_cell_list_uneven_ions_vs_oracle(oracle_lib, precision, shape):
         x0[:, 0] = 0.05 * lam + 0.01 * lam * rng.uniform(size=len(x0))
         x0[:, 1] = 0.05 * lam + 0.01 * lam * rng.uniform(size=len(x0))
     say("cell list, uneven ions", shape, precision)
-    _check(oracle_lib, cfg, x0, precision)
+    fc = _check(oracle_lib, cfg, x0, precision)
+    assert 0 < fc["units"] <= fc["capacity"]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+@pytest.mark.parametrize("rs", [None, 0.8])
+def test_cell_list_overflow_falls_back_to_the_older_kernels(oracle_lib, precision, rs):
+    """20000 ions in a ball of half the cutoff make more units than the buffer
+    holds: k_pair_cell (FP64) or k_pair32_symcol (FP32c) computes the force on
+    the list's grid, hard and switched.  Spread out again, the same context
+    runs the list, and a step from the packed state matches the oracle's."""
+    from oracle.oracle import fp32c_rounded_positions
+
+    from opendust_amd import engine
+
+    cfg, x0, v0 = _setup(20000, precision, 1.0, rs, R=3.0, H=30.0)
+    packed = _ball(cfg, len(x0), np.random.RandomState(6))
+    say("cell list, overflow", precision, "rs", rs)
+    fc = _check(oracle_lib, cfg, packed, precision)
+    assert fc["units"] > fc["capacity"] > 0
+    with engine.Engine(cfg) as e:
+        e.set_ions(packed, v0)
+        e.run(1)
+        fc = e.force_cells()
+        x, v = e.get_ions()
+        fl, _, _ = e.step_info()
+        assert fc["units"] > fc["capacity"]
+        assert np.all(fc["cell"][fl != 0] == np.prod(fc["dims"]))  # flagged ions are left out
+        e.set_ions(x0, v0)
+        fc = e.force_cells()
+        assert 0 < fc["units"] <= fc["capacity"]
+    q0 = np.array([cfg.dust_q0[0]])
+    xo, vo, _, _, flo, _ = oracle_lib.step(cfg, packed, v0, q0, 0)
+    assert np.array_equal(fl, flo)
+    if precision == "fp64":
+        assert np.max(np.abs(x - xo)) <= 1e-11 * cfg.R and np.max(np.abs(v - vo)) <= 1e-10 * np.max(np.abs(vo))
+    else:
+        # kept ions: the drift of the force error, the rounding of the positions and its arithmetic
+        f, fr = (oracle_lib.pair_forces(cfg, p) for p in (packed, fp32c_rounded_positions(cfg, packed)))
+        fn = np.linalg.norm(f, axis=1)
+        f_cut = oracle_lib.cut_force_at_cutoff(cfg) if rs is None else 0.0
+        edge = oracle_lib.cut_edge_count(cfg, packed, 1e-6)
+        err = np.linalg.norm(fr - f, axis=1) + 1e-5 * fn + 1e-6 * np.sqrt(np.mean(fn ** 2)) + edge * f_cut
+        bound = err * cfg.dt * cfg.dt / 2 / cfg.m_s + 1e-12 * cfg.R
+        keep = fl == 0
+        assert np.all(np.linalg.norm(x - xo, axis=1)[keep] <= bound[keep])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+def test_cell_list_beyond_16_bit_ids(precision):
+    """A grid of the list with more than 65536 cells: three radix passes, the
+    device's binning and order bit-exact."""
+    from opendust_amd import engine
+
+    cfg, x0, _ = _setup(300000, precision, 1.0, None, R=10.0, H=40.0)
+    say("cell list, many cells", precision)
+    with engine.Engine(cfg) as e:
+        e.pair_forces(x0)
+        fc = e.force_cells()
+    nx, ny, nz = fc["dims"]
+    say("  grid", fc["dims"], "radix passes", fc["radix_passes"])
+    assert nx * ny * nz > 65536 and fc["radix_passes"] == 3 and 0 < fc["units"] <= fc["capacity"]
+    w, h = fc["size"]
+    ix, iy = (np.clip(np.floor((x0[:, k] + cfg.R) / w), 0, nx - 1).astype(int) for k in (0, 1))
+    want = np.clip(np.floor((x0[:, 2] + cfg.H / 2) / h), 0, nz - 1).astype(int) + nz * (ix + nx * iy)
+    assert np.array_equal(fc["cell"], want)
+    assert np.array_equal(fc["order"], np.lexsort((np.arange(len(want)), want)))

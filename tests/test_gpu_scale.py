@@ -155,9 +155,10 @@ def test_cutoff_cell_variants_vs_oracle(oracle_lib, rc, rs):
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 def test_cutoff_many_cells_vs_oracle(oracle_lib, precision):
-    """A grid of 40 x 40 x 80 = 128000 cells (R = 10, H = 40 r_D_e, cutoff 1
-    r_D_e), more than 16-bit cell ids hold (three radix passes): binning and
-    order bit-exact, forces as in the dense case."""
+    """A cutoff/4 grid of more cells than 16-bit ids hold (R = 10, H = 40 r_D_e,
+    cutoff 1 r_D_e): the cells and order that od_get_cells reports bit-exact,
+    forces as in the dense case.  (The forces' own grid and its radix passes:
+    test_gpu_cell_list.py.)"""
     eng = _eng()
     od, cfg, x0, v0 = _dense_setup(precision, 1.0, None, N=20000, R=10.0, H=40.0, seed=2, np_seed=3)
     say("many cells", precision, "N", cfg.n_ions)
