@@ -352,7 +352,11 @@ struct od_ctx {
   int list = 0, cl_cap = 0, n_entries = 0, item_len = 64, cl_chain = 64;
   CellGrid grid;
   int n_set = 0;                  // forward column offsets + 1
-  uint32_t* rc4_cell = nullptr;   // od_get_cells' cells, where the grid is another
+  // od_get_cells' cells, where the grid is another, and where they come from:
+  // the state's positions with (CELLS_KEPT) or without the flagged ions left
+  // out, or binned already (od_pair_forces)
+  uint32_t* rc4_cell = nullptr;
+  enum { CELLS_STATE, CELLS_KEPT, CELLS_BINNED } cells_from = CELLS_STATE;
   int2* cl_rng = nullptr;
   int *cl_cnt = nullptr, *cl_u0 = nullptr, *cl_total = nullptr;
   double* cl_tp = nullptr;
@@ -1314,8 +1318,7 @@ template <class T>
 static int build_cells_t(od_ctx* c, const double* X, const uint32_t* flags, const void* pos) {
   using PV = typename Pos<T>::V;
   const int np = c->n_pad, nb = c->nb, nc = c->n_cells;
-  hipLaunchKernelGGL(k_bin, dim3(nb), dim3(256), 0, c->stream, c->dP, X, flags, c->ckey[0], c->cval[0],
-                     c->rc4_cell);
+  hipLaunchKernelGGL(k_bin, dim3(nb), dim3(256), 0, c->stream, c->dP, X, flags, c->ckey[0], c->cval[0]);
   for (int pass = 0; pass < c->rs_passes; ++pass) {
     const int in = pass & 1, out = 1 - in, shift = 8 * pass;
     hipLaunchKernelGGL(k_rs_hist, dim3(c->rs_nblk), dim3(256), 0, c->stream, c->ckey[in], np, shift, c->rs_nblk,
@@ -1539,6 +1542,7 @@ extern "C" int od_set_ions(od_ctx* c, const double* x, const double* v, int64_t 
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->stream));
   c->have_ions = true;
+  c->cells_from = od_ctx::CELLS_STATE;
   return OD_OK;
 }
 
@@ -1707,6 +1711,7 @@ extern "C" int od_run(od_ctx* c, int64_t nsteps, od_dust_record* out, int32_t fl
     HIPCHK(hipStreamSynchronize(c->stream));
     c->host_step += chunk;
     done += chunk;
+    c->cells_from = od_ctx::CELLS_KEPT;
     if (herr) return set_err(OD_ERR_NONFINITE, "non-finite ion position or velocity before step %lld",
                              (long long)c->host_step);
   }
@@ -1749,7 +1754,13 @@ extern "C" int od_get_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sorted_ion
   fill_params(&c->cfg, c->n_pad, &hp);
   const uint32_t n_cells = (uint32_t)hp.rc4_cells;
   if (c->rc4_cell) {
-    // the forces' grid is another: (cell, ion) order of the binned ions
+    // the forces' grid is another: (cell, ion) order of the binned ions.  A step
+    // moves only flagged ions after its force evaluation.
+    if (c->cells_from != od_ctx::CELLS_BINNED) {
+      hipLaunchKernelGGL(k_rc4_cells, dim3(c->nb), dim3(256), 0, c->stream, (const DevParams*)c->dP,
+                         (const double*)c->X, c->cells_from == od_ctx::CELLS_KEPT ? c->flags : nullptr, c->rc4_cell);
+      HIPCHK(hipGetLastError());
+    }
     std::vector<uint32_t> cell(c->n_pad);
     HIPCHK(hipMemcpyAsync(cell.data(), c->rc4_cell, c->n_pad * 4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -2007,6 +2018,11 @@ extern "C" int od_pair_forces(od_ctx* c, const double* x, double* f) {
   if (e == hipSuccess) {
     rc = load_positions(c, dX, pi, pj);
     if (rc == OD_OK) rc = launch_forces(c, dX, pj, nullptr, dF, false);
+    if (c->rc4_cell) {
+      hipLaunchKernelGGL(k_rc4_cells, dim3(c->nb), dim3(256), 0, c->stream, (const DevParams*)c->dP, (const double*)dX,
+                         (const uint32_t*)nullptr, c->rc4_cell);
+      c->cells_from = od_ctx::CELLS_BINNED;
+    }
     e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(sf.data(), dF, sf.size() * 8, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);

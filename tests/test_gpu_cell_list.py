@@ -239,6 +239,46 @@ def test_cell_list_overflow_falls_back_to_the_older_kernels(oracle_lib, precisio
         assert np.all(np.linalg.norm(x - xo, axis=1)[keep] <= bound[keep])
 
 
+def test_cells_of_every_kind_of_evaluation(oracle_lib):
+    """od_get_cells, which bins on request, after forces of other positions, of
+    a new state and of a step (reinjected ions left out)."""
+    from opendust_amd import engine
+
+    cfg, x0, v0 = _setup(5000, "fp32c", 1.5, None, R=3.0, H=6.0)
+    x0[:9, 2] = 0.51 * cfg.H
+    y = x0 * 0.7
+
+    def want(x, left_out=None):
+        cell = np.array([oracle_lib.cell_of(cfg, xi)[0] for xi in x])
+        dims = oracle_lib.cell_of(cfg, x[0])[1]
+        if left_out is not None:
+            cell[left_out] = np.prod(dims)
+        order = np.lexsort((np.arange(len(cell)), cell))
+        return cell, order[: int(np.sum(cell < np.prod(dims)))], dims
+
+    def same(got, ref):
+        return np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1]) and got[2] == ref[2]
+
+    say("cells of every kind of evaluation")
+    with engine.Engine(cfg) as e:
+        e.set_ions(x0, v0)
+        assert same(e.cells(), want(x0))
+        e.pair_forces(y)
+        assert same(e.cells(), want(y))
+        for flags in (0, engine.RUN_GRAPH):
+            e.run(5, flags)
+            fl, _, n_re = e.step_info()
+            assert same(e.cells(), want(e.get_ions()[0], fl != 0))
+        e.run(0)
+        assert same(e.cells(), want(e.get_ions()[0], fl != 0))
+        e.set_ions(x0, v0)
+        assert same(e.cells(), want(x0))
+        e.run(1)
+        fl, _, n_re = e.step_info()
+        assert n_re >= 9
+        assert same(e.cells(), want(e.get_ions()[0], fl != 0))
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 def test_cell_list_beyond_16_bit_ids(precision):
     """A grid of the list with more than 65536 cells: three radix passes, the
