@@ -94,6 +94,43 @@ def test_batch_one_step_vs_oracle(oracle_lib, precision):
     b.close()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+def test_batch_row_items_vs_oracle(oracle_lib, precision):
+    """pair_mode = PAIR_ROWS on a batch: the item kernel (512 targets by 8192
+    sources) and its reduction, which the automatic choice leaves to batches
+    whose wave tiles do not fit.  One simulation with more than one source
+    chunk; velocities after a step carry the force."""
+    import contextlib
+    import io
+
+    from opendust_amd import engine, sweep, workloads
+
+    with contextlib.redirect_stdout(io.StringIO()):
+        ods = [workloads.single_dust(N=n, n=10, precision=precision, seed=61 + i) for i, n in enumerate((700, 9000, 2048))]
+    np.random.seed(12)
+    cfgs, states = sweep.prepare_batch(ods, device=0, alphas=[workloads.synthetic_alpha(od) for od in ods])
+    say("batch row items", precision, [c.n_ions for c in cfgs])
+    out = {}
+    for mode in (engine.PAIR_ROWS, engine.PAIR_AUTO):
+        for c in cfgs:
+            c.pair_mode = mode
+        with engine.Batch(cfgs) as b:
+            for s, (x0, v0) in enumerate(states):
+                b.set_ions(s, x0, v0)
+            b.run(1)
+            out[mode] = [b.get_ions(s) for s in range(len(cfgs))]
+    for s, (cfg, (x0, v0)) in enumerate(zip(cfgs, states)):
+        x_g, v_g = out[engine.PAIR_ROWS][s]
+        x_o, v_o, _, _, _, _ = oracle_lib.step(cfg, x0, v0, _q0(cfg), 0)
+        dx = np.max(np.abs(x_g - x_o)) / cfg.R
+        dv = np.max(np.abs(v_g - v_o)) / np.max(np.abs(v_o))
+        say("  sim", s, "N", cfg.n_ions, "max |dx|/R", dx, "max |dv|/max|v|", dv)
+        assert dx <= (1e-11 if precision == "fp64" else 1e-6)
+        assert dv <= (1e-10 if precision == "fp64" else 1e-4)
+    # another kernel than the automatic one: the last bits differ
+    assert any(not np.array_equal(a[1], b[1]) for a, b in zip(out[engine.PAIR_ROWS], out[engine.PAIR_AUTO]))
+
+
 def test_batch_multi_step_fp64_vs_oracle(oracle_lib):
     from opendust_amd import engine
 
