@@ -93,15 +93,12 @@ STAGE_BYTES_PER_ION = {
 STAGE_BYTES_PER_ION_CUTOFF = dict(STAGE_BYTES_PER_ION, kick2=141, inflow=4)
 
 
-def cell_stage_bytes_per_ion(n_cells):
+def cell_stage_bytes_per_ion(passes):
     """Binning (read X 24 + flags 4, write key and value 8), one 8-bit radix
     pass per digit of the cell ids (read key 4 for the histogram, read and
     write key and value 16), gather (read key, value 8 and the position 16,
     write the sorted position 16)."""
-    passes = 1
-    while passes < 4 and (n_cells >> (8 * passes)) != 0:
-        passes += 1
-    return 36 + 20 * passes + 40, passes
+    return 36 + 20 * passes + 40
 
 
 def hbm_stages(stage_ms, n_ions, bytes_per_ion):
@@ -206,12 +203,11 @@ def cutoff_leg(steps):
     wall = time.perf_counter() - t0
     ms, nl = e.pair_timing()
     in_range, cand = e.cutoff_pair_count()
-    _, _, dims = e.cells()
+    cells = e.force_cells()
     e.run(2, engine.RUN_PROFILE_STAGES)
     st, _ = e.stage_timing()
     e.close()
-    n_cells = dims[0] * dims[1] * dims[2]
-    cb, passes = cell_stage_bytes_per_ion(n_cells)
+    cb = cell_stage_bytes_per_ion(cells["radix_passes"])
     return {
         "workload": "single dust, 2^22 superions, R=10 r_D_e, H=20 r_D_e, hard cutoff 2 r_D_e, cell list rebuilt "
                     "every step",
@@ -224,11 +220,12 @@ def cutoff_leg(steps):
         "cell_kernel_tflops_alg": in_range * FLOP_PER_PAIR / (ms / max(nl, 1) * 1e-3) / 1e12,
         "cell_kernel_frac_of_fp32_peak": in_range * FLOP_PER_PAIR / (ms / max(nl, 1) * 1e-3) / 1e12
                                          / FP32_PEAK_TFLOPS,
-        # variant 0: the evenly split cell list (its own grid; "grid" is od_get_cells')
+        # variant 0: the evenly split cell list
         "cell_kernel_variant": {"sym_tile": variant,
                                 "targets_per_lane": {0: 2, 1: 1, 2: 2, 3: 4, 4: 1, 5: 2, 6: 4}.get(variant),
                                 "sources_from_lds": variant in (0, 4, 5, 6)},
-        "grid": {"dims": list(dims), "cells": n_cells, "radix_passes": passes},
+        "grid": {"dims": list(cells["dims"]), "cells": int(np.prod(cells["dims"])),
+                 "radix_passes": cells["radix_passes"]},
         "stage_ms": st,
         "hbm_stages": hbm_stages(st, 2 ** 22, dict(STAGE_BYTES_PER_ION_CUTOFF, cells=cb)),
     }
@@ -488,7 +485,7 @@ def main():
                             if (mode == engine.PAIR_SYM and N == 2 ** 20 and tile) else (None, None))
     log("fp32c: %.2f ms/step, pair kernel %.2f ms, %.3e pairs/s" % (ms_per_step, kernel_ms, value))
 
-    # plain FP64 GPU path (every ordered pair, the row kernel), the automatic FP64 kernel, and the
+    # FP64 as a caller gets it, the plain FP64 row kernel (every ordered pair) beside it, and the
     # FP32c-vs-FP64 dust force error from the same state
     fp64 = None
     if args.fp64_steps > 0:
@@ -497,7 +494,7 @@ def main():
         rows64 = engine.Config.from_buffer_copy(cfg64)
         rows64.pair_mode = engine.PAIR_ROWS
         res = {}
-        for prec, c in (("fp64", rows64), ("fp64_auto", cfg64), ("fp32c", cfg)):
+        for prec, c in (("fp64", cfg64), ("fp64_rows", rows64), ("fp32c", cfg)):
             e = engine.Engine(c)
             e.set_ions(x_mid, v_mid)
             e.set_dust_charges(q_mid)
@@ -515,8 +512,9 @@ def main():
             "ms_per_step": t64 / args.fp64_steps * 1e3,
             "pair_interactions_per_s": pairs_step * args.fp64_steps / t64,
             "fp32c_speedup": value / (pairs_step * args.fp64_steps / t64),
-            "auto_ms_per_step": res["fp64_auto"][0] / args.fp64_steps * 1e3,
-            "auto_pair_interactions_per_s": pairs_step * args.fp64_steps / res["fp64_auto"][0],
+            "rows_ms_per_step": res["fp64_rows"][0] / args.fp64_steps * 1e3,
+            "rows_pair_interactions_per_s": pairs_step * args.fp64_steps / res["fp64_rows"][0],
+            "fp32c_speedup_vs_fp64_rows": value / (pairs_step * args.fp64_steps / res["fp64_rows"][0]),
             "dust_force_rel_err_first_step": float(np.linalg.norm(fo32 - fo64) / np.linalg.norm(fo64)),
         }
         log("fp64:", fp64)
