@@ -145,9 +145,8 @@ __device__ __forceinline__ double recip64(double b) {
   return fma(z, fma(e, e, e), z);
 }
 
-__device__ __forceinline__ double exp2_neg64(double r) {
-  const double n = __builtin_rint(-r);
-  const double f = -r - n;
+// 2^(n + f): n integral, |f| <= 1/2
+__device__ __forceinline__ double exp2_64(double n, double f) {
   double q = 0x1.e9d3fe3952179p-32;
   q = fma(q, f, 0x1.e6063f7217bc6p-28);
   q = fma(q, f, 0x1.b524fae627834p-24);
@@ -163,6 +162,19 @@ __device__ __forceinline__ double exp2_neg64(double r) {
   int i;
   asm("v_cvt_i32_f64 %0, %1" : "=v"(i) : "v"(n));
   return __builtin_amdgcn_ldexp(q, i);
+}
+
+__device__ __forceinline__ double exp2_neg64(double r) {
+  const double n = __builtin_rint(-r);
+  return exp2_64(n, -r - n);
+}
+
+// exp(-d): n + f = -d log2 e with the roundings of f alone (log2 e in two parts:
+// one double is off by 1.4e-17 of its value, a bias of d times that)
+__device__ __forceinline__ double exp_neg64(double d) {
+  constexpr double L = 1.4426950408889634, L_lo = 2.0355273740931033e-17;
+  const double n = __builtin_rint(-d * L);
+  return exp2_64(n, fma(-d, L_lo, fma(-d, L, -n)));
 }
 
 // sqrt(r2), r2 >= 1e-300: the rsqrt seed's third-order step on r = r2 y
