@@ -2261,8 +2261,9 @@ extern "C" int od_tune(od_ctx* c, int32_t reps, int32_t* sym_chunk, int32_t* sym
   if (!c) return set_err(OD_ERR_ARG, "null context");
   if (reps < 1 || reps > 100) return set_err(OD_ERR_ARG, "reps %d outside [1, 100]", reps);
   int chosen = 0, var = -1;
+  if (c->cut && c->prec == OD_PREC_FP32C && !c->have_ions)
+    return set_err(OD_ERR_STATE, "od_tune needs the ions (call od_set_ions first)");
   if (c->cut && c->prec == OD_PREC_FP32C && !c->list) {
-    if (!c->have_ions) return set_err(OD_ERR_STATE, "od_tune needs the ions (call od_set_ions first)");
     HIPCHK(hipSetDevice(c->dev));
     CHKRET(tune_cells(c, reps, &var));
     CHKRET(load_positions(c, c->X, c->pi, c->pj));

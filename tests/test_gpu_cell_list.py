@@ -298,3 +298,22 @@ def test_cell_list_beyond_16_bit_ids(precision):
     want = np.clip(np.floor((x0[:, 2] + cfg.H / 2) / h), 0, nz - 1).astype(int) + nz * (ix + nx * iy)
     assert np.array_equal(fc["cell"], want)
     assert np.array_equal(fc["order"], np.lexsort((np.arange(len(want)), want)))
+
+
+def test_tune_of_a_cutoff_context():
+    """od_tune on a cutoff context: refused before there are ions, whatever
+    kernel it runs; nothing to tune for the list, a variant for the others."""
+    from opendust_amd import engine
+
+    cfg, x0, v0 = _setup(3000, "fp32c", 2.0, None)
+    for tile in (0, 2):
+        cfg.sym_tile = tile
+        say("tune of a cutoff context, sym_tile", tile)
+        with engine.Engine(cfg) as e:
+            with pytest.raises(RuntimeError, match="needs the ions"):
+                e.tune(1)
+            e.set_ions(x0, v0)
+            chosen = e.tune(1)
+            assert chosen == (0, 0) if tile == 0 else chosen[0] == 0 and 1 <= chosen[1] <= 6
+            assert e.sym_choice() == chosen
+            e.run(2)
