@@ -851,7 +851,8 @@ static double cell_list_units(const od_config* cfg, int n, CellGrid g) {
 // 130001 ions FP64 1.30 -> 0.47 ms (pair terms per in-range pair 15.9 ->
 // 5.4), FP32c 32768 ions 0.24 -> 0.06, 262144 1.07 -> 0.55, 2^20 5.6 -> 5.0
 // (with the pairs out of range skipped and cl_waves 0.39, 0.05, 0.46 and 3.8);
-// at 2^22 the choice is columns of cutoff/4.
+// at 2^22 the choice is columns of cutoff/4.  The cost is a model: at 2^18 it
+// takes columns of one cutoff (475 us) where half of that measured 451.
 // Grids of more cells than half the ions (or 65536) are left out: false if none
 // remains, where the ions are so thin that most cells are empty whatever the
 // grid, entries outnumber ions many times, and the older kernels are faster
@@ -926,6 +927,10 @@ static int chain_steps(const od_config* cfg, int n) {
 // Whether the context runs k_cell_list, and its grid: where choose_grid has one
 // and the partials, at twice the even spread's units, fit CELL_LIST_MAX_BYTES,
 // unless the configuration fixes a variant of k_pair32_symcol.
+// 24e9: 2^22 ions at 667 per r_D_e^3 take 23.7 GB, the largest run measured
+// (43.1 ms per step against 54.6 with the older kernels, whose 5.9 GB no bound
+// stops).  The partials grow as ions times density; past the bound the older
+// kernels run at their own pace (FP64 already between 2^21 and 2^22 ions).
 constexpr double CELL_LIST_MAX_BYTES = 24e9;
 // below COUNT_MAX, so a unit count that saturated is over every capacity
 constexpr int CELL_LIST_MAX_UNITS = 1000000000;
@@ -1039,9 +1044,12 @@ static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
 
 // Whether a configuration without a schedule of its own runs the wave tiles:
 // FP64 whenever their partials fit; FP32 below TILE_FP32_SUBS sub-blocks of
-// 64 ions per simulation, above which the row groups of k_pair32_sym are
-// faster.  A configuration that fixes source chunks (j_split), blocks per
-// work-group, a variant or bands keeps the kernels those belong to.
+// 64 ions per simulation.  Step, ms, tiles and k_pair32_sym at its default
+// schedule: 131072 ions 4.66 and 4.73, 200000 10.6 and 11.5, 2^18 18.17 and
+// 18.23, 300000 23.7 and 23.7, 400000 42.1 and 42.0, 2^19 71.9 and 70.5, 2^20
+// 285 and 274: level from 2^18, where the blocks write fewer partials.  A
+// configuration that fixes source chunks (j_split), blocks per work-group, a
+// variant or bands keeps the kernels those belong to.
 constexpr int TILE_FP32_SUBS = 4096;
 static bool tile_chosen(const od_config* cfg, const TileSims& sims) {
   const bool fp32 = cfg->precision == OD_PREC_FP32C;
