@@ -350,6 +350,7 @@ struct od_ctx {
   void* spos = nullptr;
   // even split of the cell list (k_cell_list): entries, first units, partials
   int list = 0, cl_cap = 0, n_entries = 0, item_len = 64, cl_chain = 64;
+  bool cl_symcol = false;         // what takes over from the list is k_pair32_symcol, else k_pair_cell
   CellGrid grid;
   int n_set = 0;                  // forward column offsets + 1
   // od_get_cells' cells, where the grid is another, and where they come from:
@@ -932,16 +933,29 @@ static int chain_steps(const od_config* cfg, int n) {
 // stops).  The partials grow as ions times density; past the bound the older
 // kernels run at their own pace (FP64 already between 2^21 and 2^22 ions).
 constexpr double CELL_LIST_MAX_BYTES = 24e9;
+// Units grow with the square of the density where ions gather, and what takes
+// over beyond the buffer is slower, so contexts for which that is cheap hold a
+// buffer for ions this many times denser than the even spread (131072 ions, r_c =
+// 2, squeezed twelvefold, FP32c: force 0.93 ms before the list, 29.4 ms with twice
+// the even spread's units, 0.93 now; 10^6 ions squeezed to z/10 15.8 before, 17.3).
+constexpr double CELL_LIST_SPARE = 16.0, CELL_LIST_SPARE_BYTES = 4e9;
+// FP32c: from columns of this p2 (cutoff/4 or less) on k_pair32_symcol takes over
+// from the list, as it does without one (2^22 ions squeezed to z/4: 129 ms, with
+// k_pair_cell 292); on wider ones k_pair_cell (131072 ions, 200 times denser: 16.7
+// ms, k_pair32_symcol 821; 10^6 ions, 12 times: 67 and 155, columns of cutoff/4 32).
+constexpr int CELL_FALL_P2 = 8;
 // below COUNT_MAX, so a unit count that saturated is over every capacity
 constexpr int CELL_LIST_MAX_UNITS = 1000000000;
 static_assert(CELL_LIST_MAX_UNITS < COUNT_MAX, "a saturated unit count must exceed the capacity");
-static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, CellGrid* g, int* cap) {
+static bool cell_list_chosen(const od_ctx* c, const od_config* cfg, CellGrid* g, int* cap, int* cap_min) {
   const bool fp32 = c->prec == OD_PREC_FP32C;
   if (fp32 && cfg->sym_tile > 0) return false;
   if (!choose_grid(cfg, c->n, g)) return false;
-  const double units = 2.0 * cell_list_units(cfg, c->n, *g) + 4096.0;
-  *cap = (int)std::min(units, (double)CELL_LIST_MAX_UNITS);
-  return units * 192.0 * (fp32 ? 4.0 : 8.0) <= CELL_LIST_MAX_BYTES;
+  const double even = cell_list_units(cfg, c->n, *g), unit_bytes = 192.0 * (fp32 ? 4.0 : 8.0);
+  const double least = 2.0 * even + 4096.0;
+  *cap_min = (int)std::min(least, (double)CELL_LIST_MAX_UNITS);
+  *cap = (int)std::max((double)*cap_min, std::min(CELL_LIST_SPARE * even, CELL_LIST_SPARE_BYTES / unit_bytes));
+  return least * unit_bytes <= CELL_LIST_MAX_BYTES;
 }
 
 // the cell list's buffers on hp's grid (c->list: with those of k_cell_list)
@@ -977,9 +991,6 @@ static int alloc_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   if ((rc = dalloc(&c->scan_tsum, n_tiles * 4)) || (rc = dalloc(&c->scan_toff, n_tiles * 4))) return rc;
   c->sc_var = CC_DEFAULT;
   const bool fp32 = c->prec == OD_PREC_FP32C;
-  const size_t b_sc = fp32 ? (size_t)c->n_set * 3 * np * 8 : 0;
-  const size_t b_tp = c->list ? ((size_t)cl_waves(c->n) + c->max_items) * 3 * CL_G * 8 : 0;
-  const size_t b_list = c->list ? b_tp + (size_t)c->cl_cap * 192 * (fp32 ? 4 : 8) : 0;
   if (c->list) {
     // one allocation for the tables
     const size_t ne = (size_t)c->n_entries + 1;
@@ -991,14 +1002,19 @@ static int alloc_cells(od_ctx* c, const od_config* cfg, const DevParams& hp) {
   // one for the partial sums: an evaluation writes either the list's or, where
   // that has no room, k_pair32_symcol's, so both lie in the same place (2^22
   // ions: 23.7 GB instead of 29.6)
+  const size_t b_sc = fp32 && (!c->list || c->cl_symcol) ? (size_t)c->n_set * 3 * np * 8 : 0;
+  const size_t b_tp = c->list ? ((size_t)cl_waves(c->n) + c->max_items) * 3 * CL_G * 8 : 0;
+  const size_t b_list = c->list ? b_tp + (size_t)c->cl_cap * 192 * (fp32 ? 4 : 8) : 0;
   if ((b_list || b_sc) && (rc = dalloc(&c->cell_sums, std::max(b_list, b_sc + b_sc / 2)))) return rc;
   if (c->list) {
     c->cl_tp = (double*)c->cell_sums;
     c->cl_sp = c->cell_sums + b_tp;
   }
-  if (fp32) {
+  if (b_sc) {
     c->sc_tp = (double*)c->cell_sums;
     c->sc_sp = (float*)(c->cell_sums + b_sc);
+  }
+  if (fp32) {
     c->sc_var = cell_variant_of(cfg->sym_tile);
     if (c->sc_var < 0) return set_err(OD_ERR_ARG, "cutoff mode: sym_tile %d outside [0, %d]", cfg->sym_tile, CC_N_VARIANTS);
   }
@@ -1026,15 +1042,21 @@ static int setup_cells(od_ctx* c, const od_config* cfg, DevParams& hp) {
                    cfg->R, cfg->H, OD_MAX_CELLS);
   c->cut = 1;
   CellGrid g;
-  c->list = cell_list_chosen(c, cfg, &g, &c->cl_cap) ? 1 : 0;
+  int cap_min = 0;
+  c->list = cell_list_chosen(c, cfg, &g, &c->cl_cap, &cap_min) ? 1 : 0;
   if (c->list) {
     c->grid = g;
     c->cl_chain = chain_steps(cfg, c->n);
+    c->cl_symcol = c->prec == OD_PREC_FP32C && g.p2 >= CELL_FALL_P2;
     fill_params(cfg, c->n_pad, &hp, g);
-    const int rc = alloc_cells(c, cfg, hp);
-    if (rc != OD_ERR_HIP && (rc != OD_OK || memory_left(c->n_pad))) return rc;
+    for (;;) {
+      const int rc = alloc_cells(c, cfg, hp);
+      if (rc != OD_ERR_HIP && (rc != OD_OK || memory_left(c->n_pad))) return rc;
+      free_cells(c);
+      if (c->cl_cap == cap_min) break;
+      c->cl_cap = cap_min;
+    }
     // the memory is short: the older kernels, on their own grid
-    free_cells(c);
     c->list = 0;
     c->grid = CellGrid();
     fill_params(cfg, c->n_pad, &hp);
@@ -1378,13 +1400,14 @@ static int launch_forces_t(od_ctx* c, const double* X, const void* pos, const ui
       if (c->cl_chain == 16) fn = sw ? k_cell_list<T, 2, 16> : k_cell_list<T, 1, 16>;
       if (c->cl_chain == 4) fn = sw ? k_cell_list<T, 2, 4> : k_cell_list<T, 1, 4>;
     }
-    hipLaunchKernelGGL(fn, dim3(cl_waves(c->n)), dim3(64), 0, c->stream, c->dP, (const PV*)c->spos, c->skey, c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries,
-                       n_units, c->cl_cap, c->cl_tp, (T*)c->cl_sp);
+    hipLaunchKernelGGL(fn, dim3(cl_waves(c->n)), dim3(64), 0, c->stream, c->dP, (const PV*)c->spos, c->skey,
+                       c->cell_start, c->items, c->cl_rng, c->cl_u0, c->n_entries, n_units, c->cl_cap, c->cl_tp,
+                       (T*)c->cl_sp);
     hipLaunchKernelGGL(k_cell_list_reduce<T>, dim3(c->n_pad / 64), dim3(64 * REDUCE_PARTS), 0, c->stream, c->dP,
                        c->skey, c->sval, c->cell_start, c->item_off, c->cl_rng, c->cl_u0, n_units, c->cl_cap, cl_waves(c->n),
                        (const double*)c->cl_tp, (const T*)c->cl_sp, F);
   }
-  if constexpr (std::is_same<T, float>::value) {
+  if (std::is_same<T, float>::value && (!c->list || c->cl_symcol)) {
     // symmetric: forward neighbour columns and the own column, per-ion reduction
     const float4* sp4 = (const float4*)c->spos;
     const dim3 g(c->n_cols * c->n_set);

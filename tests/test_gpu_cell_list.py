@@ -103,35 +103,40 @@ def test_sparse_cylinder_keeps_the_older_kernels(oracle_lib, precision):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
-def test_short_memory_steps_down_to_the_older_kernels(precision):
-    """2^20 ions at r_c = 2 in R = 10, H = 20 on a GPU with less free memory
-    than the list wants: the older kernels on their own grid, the same forces
-    up to rounding (FP32c: and up to pairs at the cutoff counted on one side,
-    each one pair force there)."""
+def test_short_memory_steps_down(precision):
+    """2^20 ions at r_c = 2 in R = 10, H = 20: the list with its 4 GB of spare
+    units; on a GPU with less free memory with fewer; with less still the older
+    kernels on their own grid.  The same forces: to the last bit with fewer
+    units, else up to rounding (FP32c: and up to pairs at the cutoff counted on
+    one side, each one pair force there)."""
     from opendust_amd import engine
 
     cfg, x0, _ = _setup(1 << 20, precision, 2.0, None, R=10.0, H=20.0)
     say("short memory, cutoff", precision)
-    before = gpu_free_bytes()
-    e = engine.Engine(cfg)
-    held = before - gpu_free_bytes()
-    say("  device memory of the context, GB:", held / 1e9)
-    f = e.pair_forces(x0)
-    assert e.sym_choice() == (0, 0)
-    e.close()
-    # beside the partial sums (FP64 4.8, FP32c 2.6 GB) under 0.3 kB per ion: the
-    # fallback kernel's lie in the same place
-    assert 2.5e9 <= held <= (5.2e9 if precision == "fp64" else 2.95e9)
-    with gpu_memory_left(int(held - 0.7e9)):
-        e = engine.Engine(cfg)
-        g = e.pair_forces(x0)
-        choice = e.sym_choice()
-        e.close()
+
+    def forces():
+        before = gpu_free_bytes()
+        with engine.Engine(cfg) as e:
+            held = before - gpu_free_bytes()
+            f = e.pair_forces(x0)
+            fc = e.force_cells()
+        say("  device memory of the context, GB:", held / 1e9, "capacity", fc["capacity"], "grid", fc["dims"])
+        return f, held, fc
+
+    f, held, full = forces()
+    assert 4e9 <= held <= 5.2e9
+    if precision == "fp32c":  # FP64 has no spare beyond twice the even spread
+        with gpu_memory_left(int(held - 0.7e9)):
+            g, _, fewer = forces()
+        assert full["units"] == fewer["units"] <= fewer["capacity"] < full["capacity"]
+        assert np.array_equal(f, g)
+    with gpu_memory_left(int(2.3e9)):
+        g, _, older = forces()
+    assert older["capacity"] == 0 and older["dims"] == (40, 40, 160)
     if precision == "fp64":
         fn = np.linalg.norm(f, axis=1)
         assert np.all(np.linalg.norm(g - f, axis=1) <= 1e-11 * fn + 1e-13 * np.sqrt(np.mean(fn ** 2)))
     else:
-        assert choice == (0, 5)
         assert np.linalg.norm(g - f) <= 1e-5 * np.linalg.norm(f)
 
 
@@ -198,15 +203,15 @@ def test_cell_list_uneven_ions_vs_oracle(oracle_lib, precision, shape):
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 @pytest.mark.parametrize("rs", [None, 0.8])
 def test_cell_list_overflow_falls_back_to_the_older_kernels(oracle_lib, precision, rs):
-    """20000 ions in a ball of half the cutoff make more units than the buffer
-    holds: k_pair_cell (FP64) or k_pair32_symcol (FP32c) computes the force on
-    the list's grid, hard and switched.  Spread out again, the same context
-    runs the list, and a step from the packed state matches the oracle's."""
+    """60000 ions in a ball of half the cutoff make more units than the buffer
+    holds: k_pair_cell computes the force on the list's grid, hard and
+    switched.  Spread out again, the same context runs the list, and a step
+    from the packed state matches the oracle's."""
     from oracle.oracle import fp32c_rounded_positions
 
     from opendust_amd import engine
 
-    cfg, x0, v0 = _setup(20000, precision, 1.0, rs, R=3.0, H=30.0)
+    cfg, x0, v0 = _setup(60000, precision, 1.0, rs, R=3.0, H=30.0)
     packed = _ball(cfg, len(x0), np.random.RandomState(6))
     say("cell list, overflow", precision, "rs", rs)
     fc = _check(oracle_lib, cfg, packed, precision)
@@ -277,6 +282,66 @@ def test_cells_of_every_kind_of_evaluation(oracle_lib):
         fl, _, n_re = e.step_info()
         assert n_re >= 9
         assert same(e.cells(), want(e.get_ions()[0], fl != 0))
+
+
+@pytest.mark.timeout(300)
+def test_cell_list_overflow_on_narrow_columns():
+    """2^22 ions gathered in a quarter of the cylinder's height: columns of
+    cutoff/4 and more units than the buffer holds, so k_pair32_symcol takes over
+    in FP32c on the list's grid; the forces of the same kernel on its own
+    (sym_tile = 5), whose slabs are higher, up to the rounding of the sums (a
+    switched cutoff: no pair is counted on one side only)."""
+    from opendust_amd import engine
+
+    cfg, x0, _ = _setup(1 << 22, "fp32c", 2.0, 1.8, R=10.0, H=20.0)
+    x0[:, 2] /= 4.0
+    say("cell list, overflow on narrow columns")
+    out = []
+    for tile in (0, 5):
+        cfg.sym_tile = tile
+        with engine.Engine(cfg) as e:
+            out.append(e.pair_forces(x0))
+            fc = e.force_cells()
+        say("  sym_tile", tile, "grid", fc["dims"], "units", fc["units"], "of", fc["capacity"])
+        assert fc["dims"][0] == 40 and (fc["units"] > fc["capacity"] > 0 if tile == 0 else fc["capacity"] == 0)
+    assert np.linalg.norm(out[0] - out[1]) <= 2e-6 * np.linalg.norm(out[1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+@pytest.mark.parametrize("squeeze", [12, 200])
+def test_squeezed_ions_are_no_slower_than_with_the_older_kernels(precision, squeeze):
+    """Ions gathered in 1/12 of the cylinder, which the list's buffer holds, and
+    in 1/200, which it does not: the pair stage of the automatic kernels against
+    that of the FP32c kernel on columns of cutoff/4 (sym_tile = 5).  Measured
+    1.1 and 2.0 times its time, FP64 3.2 and 4.6 (its law's rate is 0.36 of
+    FP32's); 37 and 100 times, FP64 10, when k_pair32_symcol or k_pair_cell took
+    over from a buffer of twice the even spread's units."""
+    from opendust_amd import engine
+
+    cfg, x0, v0 = _setup(131072, precision, 2.0, None, R=10.0, H=20.0)
+    x0[:, 2] /= squeeze / 4 if squeeze == 12 else squeeze / 16
+    x0[:, :2] /= 2.0 if squeeze == 12 else 4.0
+
+    def pair_ms(cfg):
+        with engine.Engine(cfg) as e:
+            e.set_ions(x0, v0)
+            best = 1e9
+            for _ in range(3):
+                e.stage_timing(True)
+                e.set_ions(x0, v0)
+                e.run(1, engine.RUN_PROFILE_STAGES)
+                best = min(best, e.stage_timing(True)[0]["pair"])
+            return best, e.force_cells()
+
+    say("squeezed ions", precision, squeeze)
+    ms, fc = pair_ms(cfg)
+    assert (fc["units"] <= fc["capacity"]) == (squeeze == 12)
+    old = engine.Config.from_buffer_copy(cfg)
+    old.precision = 0
+    old.sym_tile = 5
+    ms_old, _ = pair_ms(old)
+    say("  pair stage, ms: automatic", ms, "columns of cutoff/4, FP32c", ms_old, "units", fc["units"], fc["capacity"])
+    assert ms <= ms_old * (7.0 if precision == "fp64" else 2.0 if squeeze == 12 else 4.0)
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
