@@ -1843,7 +1843,7 @@ extern "C" int od_get_force_cells(od_ctx* c, int32_t* cell_of_ion, int32_t* sort
 
 // Ordered pair terms the context's cell kernel evaluates on a cell list
 // (cs: cell starts, key: sorted cell ids), padding lanes and slots included:
-// the FP64 kernel evaluates 64 lanes x every source of the 77 slab ranges of
+// the ordered kernel evaluates 64 lanes x every source of the slab ranges of
 // each 64-target chunk; the symmetric FP32 kernel's slots each give two
 // ordered terms (force and reaction), its own-group tiles one.
 static int64_t cell_candidates(const od_ctx* c, const std::vector<int>& cs, const std::vector<uint32_t>& key) {
